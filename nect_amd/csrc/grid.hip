@@ -10,50 +10,9 @@
 #include <cmath>
 #include <type_traits>
 
-#include "grid.hpp"
-#include "sampler.hpp"
+#include "sources.hpp"
 
 namespace nect {
-
-// ----------------------------------------------------------- position sources
-
-template <int D>
-struct PointSource {
-    const float *x;
-    int64_t n;
-    int64_t stride;
-    // 0: no such slot, 1: live slot without a sample, 2: sample.
-    __device__ __forceinline__ int get(int64_t s, float (&p)[D]) const {
-        if (s >= n) return 0;
-        const float *r = x + s * stride;
-#pragma unroll
-        for (int d = 0; d < D; ++d) p[d] = r[d];
-        return 2;
-    }
-};
-
-// Samples of the fused training path: slot 32*tile + j of the tile list.
-template <int D>
-struct RaySource {
-    const NectRay *rays;
-    const int32_t *tile_offsets;
-    const int32_t *tile_ray;
-    const int32_t *n_tiles;
-    float t;  // 4th coordinate (time) for D == 4
-    __device__ __forceinline__ int get(int64_t slot, float (&p)[D]) const {
-        const int64_t tile = slot / kTile;
-        if (tile >= n_tiles[0]) return 0;
-        const int r = tile_ray[tile];
-        const int i = (int)(tile - tile_offsets[r]) * kTile + (int)(slot % kTile);
-        const NectRay d = rays[r];
-        float q[3];
-        const bool ok = ray_sample(d, i, q);
-#pragma unroll
-        for (int k = 0; k < D && k < 3; ++k) p[k] = q[k];
-        if (D == 4) p[D - 1] = t;
-        return ok ? 2 : 1;
-    }
-};
 
 // ------------------------------------------------------------------- kernels
 
@@ -72,14 +31,19 @@ __global__ __launch_bounds__(256) void k_grid_index(NectGridDesc g, const float 
     float f[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) grid_pos(g.scale[l], xs[d], c[d], f[d]);
+    const LevelIndex<D> li = level_index<D>(g.resolution[l], g.level_size[l]);
+    uint32_t ct[D];
+    corner_terms<D>(li, c, ct);
     const int64_t base = t << D;
 #pragma unroll
-    for (int k = 0; k < (1 << D); ++k) {
-        uint32_t idx;
-        float w;
-        grid_corner<D>(g.resolution[l], g.level_size[l], c, f, k, idx, w);
-        index[base + k] = idx;
-        weight[base + k] = w;
+    for (int cx = 0; cx < 2; ++cx) {
+        uint32_t idx[1 << (D - 1)];
+        corner_entries<D>(li, ct, cx, idx);
+#pragma unroll
+        for (int q = 0; q < (1 << (D - 1)); ++q) {
+            index[base + cx + 2 * q] = idx[q];
+            weight[base + cx + 2 * q] = corner_weight<D>(f, cx | (q << 1));
+        }
     }
 }
 
@@ -268,6 +232,7 @@ __device__ __forceinline__ void backward_quad_tile(const NectGridDesc &g, const 
         const int l = GROUPED ? group_level(grp, jl, n_groups) : jl;
         if (l >= g.n_levels) break;
         const LevelInfo lv = level_info(g, l);
+        const LevelIndex<D> li = level_index<D>(lv.res, lv.size);
         float *lvl = grad + (size_t)lv.offset * F + fq * FH;
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
@@ -275,6 +240,8 @@ __device__ __forceinline__ void backward_quad_tile(const NectGridDesc &g, const 
             float f[D];
 #pragma unroll
             for (int d = 0; d < D; ++d) grid_pos(lv.scale, p[r][d], c[d], f[d]);
+            uint32_t ct[D];
+            corner_terms<D>(li, c, ct);
             bool head = m == 0 || live[r] != prev_live[r];
 #pragma unroll
             for (int d = 0; d < D; ++d) head |= (uint32_t)__shfl_up((int)c[d], 4, kWave) != c[d];
@@ -288,11 +255,11 @@ __device__ __forceinline__ void backward_quad_tile(const NectGridDesc &g, const 
                 const uint64_t after = bit == kWave - 1 ? 0ull : heads & (~0ull << (bit + 1));
                 end = after ? (__builtin_ctzll(after) >> 2) - 1 : 15;
             }
+            uint32_t idx[1 << (D - 1)];
+            corner_entries<D>(li, ct, cx, idx);
 #pragma unroll
             for (int q = 0; q < (1 << (D - 1)); ++q) {
-                uint32_t idx;
-                float w;
-                grid_corner<D>(lv.res, lv.size, c, f, cx | (q << 1), idx, w);
+                const float w = corner_weight<D>(f, cx | (q << 1));
                 float v[FH];
 #pragma unroll
                 for (int j = 0; j < FH; ++j) v[j] = w * gv[j];
@@ -300,7 +267,7 @@ __device__ __forceinline__ void backward_quad_tile(const NectGridDesc &g, const 
 #pragma unroll
                     for (int j = 0; j < FH; ++j) v[j] = run_sum_quad(v[j], m, end);
                 }
-                add_corner_pair<F>(lvl, idx, v, head && live[r], lane);
+                add_corner_pair<F>(lvl, idx[q], v, head && live[r], lane);
             }
         }
     }
@@ -399,34 +366,6 @@ struct AggPlan {
     // over, e.g., (y, x, t) has its own map)
     uint32_t cmap;
 };
-
-// dL/dfeatures as the grouped scatter reads it: rows of `stride` elements of
-// `dtype` (NECT_F32, NECT_F16 or NECT_BF16), each value multiplied by *scale
-// when scale is set (a 16-bit network backward's scaled gradient and the
-// reciprocal of its power-of-two scale: the products are exact, so the values
-// equal those of the unscaled float32 copy, which is then never written).
-struct DoutView {
-    const void *p;
-    int64_t stride;
-    int32_t dtype;
-    const float *scale;
-};
-
-__device__ __forceinline__ float dout_at(const DoutView &d, float sc, int64_t i) {
-    if (d.dtype == NECT_F16) return (float)static_cast<const _Float16 *>(d.p)[i] * sc;
-    if (d.dtype == NECT_BF16) return to_f32(static_cast<const bf16_t *>(d.p)[i]) * sc;
-    return static_cast<const float *>(d.p)[i] * sc;
-}
-
-// The grid input of a sample at (z, y, x) = q and time t under the column map.
-template <int D>
-__device__ __forceinline__ void place_sample(uint32_t cmap, const float (&q)[3], float t, float (&p)[D]) {
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-        const uint32_t k = ((cmap >> (2 * d)) & 3u) ^ (uint32_t)d;
-        p[d] = k == 0 ? q[0] : (k == 1 ? q[1] : (k == 2 ? q[2] : t));
-    }
-}
 
 // One step of the run sums along a ray in the one-lane-per-sample layout: lane
 // i adds the values of lane i + OFF of its row when `add`.  ROWS: read them
@@ -551,6 +490,9 @@ __global__ __launch_bounds__(256, MODE != 0 ? 4 : 1) void k_grid_backward_groups
         float f[D];
 #pragma unroll
         for (int d = 0; d < D; ++d) grid_pos(lv.scale, p[d], c[d], f[d]);
+        const LevelIndex<D> li = level_index<D>(lv.res, lv.size);
+        uint32_t ct[D];
+        corner_terms<D>(li, c, ct);
         bool head = !runs || m == 0 || live != prev_live;
         if (runs) {
 #pragma unroll
@@ -563,11 +505,11 @@ __global__ __launch_bounds__(256, MODE != 0 ? 4 : 1) void k_grid_backward_groups
             const uint64_t after = bit == kWave - 1 ? 0ull : heads & (~0ull << (bit + 1));
             end = after ? (__builtin_ctzll(after) >> 2) - 1 : 15;
         }
+        uint32_t idx[1 << (D - 1)];
+        corner_entries<D>(li, ct, cx, idx);
 #pragma unroll
         for (int qq = 0; qq < (1 << (D - 1)); ++qq) {
-            uint32_t idx;
-            float w;
-            grid_corner<D>(lv.res, lv.size, c, f, cx | (qq << 1), idx, w);
+            const float w = corner_weight<D>(f, cx | (qq << 1));
             float v[FH];
 #pragma unroll
             for (int jj = 0; jj < FH; ++jj) v[jj] = w * gv[jj];
@@ -575,7 +517,7 @@ __global__ __launch_bounds__(256, MODE != 0 ? 4 : 1) void k_grid_backward_groups
 #pragma unroll
                 for (int jj = 0; jj < FH; ++jj) v[jj] = run_sum_quad(v[jj], m, end);
             }
-            add_corner_pair<F>(grad + (int64_t)lv.offset * F + fq * FH, idx, v, head && live, lane);
+            add_corner_pair<F>(grad + (int64_t)lv.offset * F + fq * FH, idx[qq], v, head && live, lane);
         }
     };
     bool direct = false;
@@ -620,6 +562,7 @@ __global__ __launch_bounds__(256, MODE != 0 ? 4 : 1) void k_grid_backward_groups
             const int R = plan.rounds[l];
             if (R <= 0) continue;
             const LevelInfo lv = level_info(g, l);
+            const LevelIndex<D> li = level_index<D>(lv.res, lv.size);
             const int span = kUnitSamples / R;
             for (int h = 0; h < kUnitSamples; h += span) {
 #pragma unroll 1
@@ -639,6 +582,8 @@ __global__ __launch_bounds__(256, MODE != 0 ? 4 : 1) void k_grid_backward_groups
                     float fr[D];
 #pragma unroll
                     for (int d = 0; d < D; ++d) grid_pos(lv.scale, pa[d], c[d], fr[d]);
+                    uint32_t ct[D];
+                    corner_terms<D>(li, c, ct);
                     // lane 16 rr (ma = 0) is a head whatever its row shift reads
                     auto prev = [&](int x) { return kRows ? row_up<1>(x) : __shfl_up(x, 1, kWave); };
                     const bool prev_live = prev((int)live) != 0;
@@ -656,14 +601,15 @@ __global__ __launch_bounds__(256, MODE != 0 ? 4 : 1) void k_grid_backward_groups
                     // then the chunk's table lookups issued together (one LDS
                     // round trip when the blocks are already in the table)
                     constexpr int K = 8;
+                    uint32_t even[1 << (D - 1)], odd[1 << (D - 1)];
+                    corner_entries<D>(li, ct, 0, even);
+                    corner_entries<D>(li, ct, 1, odd);
 #pragma unroll
                     for (int k0 = 0; k0 < (1 << D); k0 += K) {
-                        uint32_t ix[K];
                         float v[K][F];
 #pragma unroll
                         for (int k = 0; k < K; ++k) {
-                            float w;
-                            grid_corner<D>(lv.res, lv.size, c, fr, k0 + k, ix[k], w);
+                            const float w = corner_weight<D>(fr, k0 + k);
 #pragma unroll
                             for (int f = 0; f < F; ++f) v[k][f] = w * gv[f];
                         }
@@ -680,7 +626,7 @@ __global__ __launch_bounds__(256, MODE != 0 ? 4 : 1) void k_grid_backward_groups
                             uint32_t key[K], hs[K], got[K];
 #pragma unroll
                             for (int k = 0; k < K; ++k) {
-                                a[k] = ((int64_t)lv.offset + ix[k]) * F;
+                                a[k] = ((int64_t)lv.offset + ((k & 1) ? odd : even)[(k0 + k) >> 1]) * F;
                                 key[k] = (uint32_t)((a[k] + lead) >> 4);
                                 hs[k] = (key[k] * 2654435761u) >> (32 - kAggLog2Slots);
                             }

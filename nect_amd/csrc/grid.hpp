@@ -77,49 +77,6 @@ __device__ __forceinline__ void grid_pos(float scale, float x, uint32_t &c, floa
     f = p - fl;
 }
 
-template <int D>
-__device__ __forceinline__ uint32_t grid_index(uint32_t res, uint32_t size, const uint32_t (&c)[D]) {
-    uint64_t stride = 1;
-    uint32_t index = 0;
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-        if (stride > size) break;
-        index += c[d] * (uint32_t)stride;
-        stride *= res;
-    }
-    if (stride > size) {
-        uint32_t h = 0;
-#pragma unroll
-        for (int d = 0; d < D; ++d) h ^= c[d] * hash_prime(d);
-        index = h;
-    }
-    return index % size;
-}
-
-// Corner k of a sample on one level: its entry (within the level) and weight.
-template <int D>
-__device__ __forceinline__ void grid_corner(uint32_t res, uint32_t size, const uint32_t (&c)[D], const float (&f)[D],
-                                            int k, uint32_t &idx, float &w) {
-    uint32_t cc[D];
-    w = 1.0f;
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-        if ((k >> d) & 1) {
-            w = w * f[d];
-            cc[d] = c[d] + 1;
-        } else {
-            w = w * (1.0f - f[d]);
-            cc[d] = c[d];
-        }
-    }
-    idx = grid_index<D>(res, size, cc);
-}
-
-template <typename T, int F>
-struct Entry {
-    T v[F];
-};
-
 // Constants of one level.
 struct LevelInfo {
     float scale;
@@ -129,6 +86,100 @@ struct LevelInfo {
 __device__ __forceinline__ LevelInfo level_info(const NectGridDesc &g, int l) {
     return LevelInfo{g.scale[l], g.resolution[l], g.level_size[l], g.offset[l]};
 }
+
+// How one level's entry index is formed (the same on every lane): dimension d
+// contributes c_d * mul[d], combined by xor on a hashed level (mul: the primes)
+// and by addition on a dense one (mul: the strides).  The reduction to the
+// level's size is a mask where the size is a power of two (every hashed level
+// nect_grid_init makes), and on the others a remainder taken only by a wave
+// that holds an index past the end (an upper corner at the far faces): a 32-bit
+// remainder by a run-time size is about 20 instructions, four of them quarter
+// rate, and was taken for every corner.  QuadCubes step (4 x 23 levels) 34.9 ->
+// 34.2 ms, 256^3 step 25.4 -> 25.1 ms.
+template <int D>
+struct LevelIndex {
+    uint32_t mul[D];
+    uint32_t size;
+    bool hashed, pow2;
+};
+
+template <int D>
+__device__ __forceinline__ LevelIndex<D> level_index(uint32_t res, uint32_t size) {
+    LevelIndex<D> li;
+    uint64_t stride = 1;
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+        li.mul[d] = (uint32_t)stride;
+        if (stride <= size) stride *= res;
+    }
+    li.hashed = stride > size;
+    if (li.hashed) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) li.mul[d] = hash_prime(d);
+    }
+    li.size = size;
+    li.pow2 = (size & (size - 1)) == 0;
+    return li;
+}
+
+// The per-dimension terms of a cell's corner 0; corner bit d adds mul[d].
+template <int D>
+__device__ __forceinline__ void corner_terms(const LevelIndex<D> &li, const uint32_t (&c)[D], uint32_t (&t)[D]) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) t[d] = c[d] * li.mul[d];
+}
+
+// Entries (within the level) of corners k = cx + 2 q, q < 2^(D-1), of the cell
+// with terms t: the corners with x-bit cx.  The level's kind is tested once, not
+// per corner, so the loads that follow stay in one block.
+template <int D>
+__device__ __forceinline__ void corner_entries(const LevelIndex<D> &li, const uint32_t (&t)[D], int cx,
+                                               uint32_t (&idx)[1 << (D - 1)]) {
+    const uint32_t t0 = t[0] + (cx ? li.mul[0] : 0u);
+    if (li.hashed) {
+#pragma unroll
+        for (int q = 0; q < (1 << (D - 1)); ++q) {
+            uint32_t i = t0;
+#pragma unroll
+            for (int d = 1; d < D; ++d) i ^= t[d] + (((q >> (d - 1)) & 1) ? li.mul[d] : 0u);
+            idx[q] = i;
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < (1 << (D - 1)); ++q) {
+            uint32_t i = t0;
+#pragma unroll
+            for (int d = 1; d < D; ++d) i += t[d] + (((q >> (d - 1)) & 1) ? li.mul[d] : 0u);
+            idx[q] = i;
+        }
+    }
+    if (li.pow2) {
+#pragma unroll
+        for (int q = 0; q < (1 << (D - 1)); ++q) idx[q] &= li.size - 1;
+    } else {
+        uint32_t most = 0;
+#pragma unroll
+        for (int q = 0; q < (1 << (D - 1)); ++q) most = max(most, idx[q]);
+        if (most >= li.size) {
+#pragma unroll
+            for (int q = 0; q < (1 << (D - 1)); ++q) idx[q] %= li.size;
+        }
+    }
+}
+
+// Weight of corner k of a cell with fractions f.
+template <int D>
+__device__ __forceinline__ float corner_weight(const float (&f)[D], int k) {
+    float w = 1.0f;
+#pragma unroll
+    for (int d = 0; d < D; ++d) w = w * (((k >> d) & 1) ? f[d] : 1.0f - f[d]);
+    return w;
+}
+
+template <typename T, int F>
+struct Entry {
+    T v[F];
+};
 
 // Level groups.  With G groups, level l belongs to group (l / G) even ? l % G
 // : G - 1 - l % G, so group g holds levels g, 2G-1-g, 2G+g, ... (for L = 16,
@@ -153,50 +204,22 @@ template <int D, int F, typename T>
 __device__ __forceinline__ void encode_half(const LevelInfo &lv, const uint32_t (&c)[D], const float (&f)[D],
                                             const T *__restrict__ table, int cx, float (&out)[F]) {
     const Entry<T, F> *lvl = reinterpret_cast<const Entry<T, F> *>(table) + lv.offset;
+    const LevelIndex<D> li = level_index<D>(lv.res, lv.size);
+    uint32_t t[D];
+    corner_terms<D>(li, c, t);
 #pragma unroll
     for (int j = 0; j < F; ++j) out[j] = 0.0f;
+    constexpr int Q = 1 << (D - 1);
+    uint32_t idx[Q];
+    corner_entries<D>(li, t, cx, idx);
+    Entry<T, F> e[Q];
 #pragma unroll
-    for (int q = 0; q < (1 << (D - 1)); ++q) {
-        uint32_t idx;
-        float w;
-        grid_corner<D>(lv.res, lv.size, c, f, cx | (q << 1), idx, w);
-        const Entry<T, F> e = lvl[idx];
+    for (int q = 0; q < Q; ++q) e[q] = lvl[idx[q]];
 #pragma unroll
-        for (int j = 0; j < F; ++j) out[j] = fmaf(w, to_f32(e.v[j]), out[j]);
-    }
-}
-
-// Interpolated features of one level (float accumulation).
-template <int D, int F, typename T>
-__device__ __forceinline__ void encode_level(const LevelInfo &lv, const float (&x)[D], const T *__restrict__ table,
-                                             float (&out)[F]) {
-    uint32_t c[D];
-    float f[D];
+    for (int q = 0; q < Q; ++q) {
+        const float w = corner_weight<D>(f, cx | (q << 1));
 #pragma unroll
-    for (int d = 0; d < D; ++d) grid_pos(lv.scale, x[d], c[d], f[d]);
-    float odd[F];
-    encode_half<D, F, T>(lv, c, f, table, 0, out);
-    encode_half<D, F, T>(lv, c, f, table, 1, odd);
-#pragma unroll
-    for (int j = 0; j < F; ++j) out[j] = out[j] + odd[j];
-}
-
-// Scatter of one level's feature gradient into the float gradient table.
-template <int D, int F>
-__device__ __forceinline__ void scatter_level(const LevelInfo &lv, const float (&x)[D], const float (&dout)[F],
-                                              float *__restrict__ grad) {
-    uint32_t c[D];
-    float f[D];
-#pragma unroll
-    for (int d = 0; d < D; ++d) grid_pos(lv.scale, x[d], c[d], f[d]);
-    float *lvl = grad + (size_t)lv.offset * F;
-#pragma unroll
-    for (int k = 0; k < (1 << D); ++k) {
-        uint32_t idx;
-        float w;
-        grid_corner<D>(lv.res, lv.size, c, f, k, idx, w);
-#pragma unroll
-        for (int j = 0; j < F; ++j) unsafeAtomicAdd(lvl + (size_t)idx * F + j, w * dout[j]);
+        for (int j = 0; j < F; ++j) out[j] = fmaf(w, to_f32(e[q].v[j]), out[j]);
     }
 }
 

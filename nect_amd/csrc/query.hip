@@ -33,10 +33,18 @@ __device__ __forceinline__ float rescale_value(const NectQueryJob &J, float mu) 
     return (float)h;
 }
 
-// Voxel (iz, iy, ix) at traversal position v of a job's grid (row order, or
-// bricks of 2^bz x 2^by x 2^bx voxels over the grid padded to whole bricks);
-// false for positions in the padding or past the grid.  The host keeps the
-// brick count below 2^31, so the brick arithmetic runs in 32 bits.
+// Voxel (iz, iy, ix) at traversal position v of a job's grid; false for positions
+// in the padding or past the grid.  Row order, or (J.brick) the grid padded to
+// whole bricks of 2^lz x 2^ly x 2^lx voxels, taken in layers of bricks stacked up
+// to 32 voxels along z; a layer column by column, a column (one stack of bricks)
+// with z fastest, then x, then y.
+// z is the grid's first coordinate, whose neighbouring cells are neighbouring
+// table entries on dense and hashed levels alike (its stride or prime is 1), so
+// a wave whose 32 voxels lie along z gathers from a fraction of the cache lines,
+// and the gathers are bound by the lines an instruction touches.  512^3 volume of
+// the 4-D BF16 model: 4 x 4 x 4 bricks one by one with x fastest 66 ms, z fastest
+// 49; stacked 8 / 16 / 32 voxels along z 38 / 33 / 29 ms.
+// The host keeps the brick count below 2^31, so the brick arithmetic runs in 32 bits.
 __device__ __forceinline__ bool query_voxel(const NectQueryJob &J, int64_t v, int32_t &iz, int32_t &iy, int32_t &ix) {
     if (J.brick == 0) {
         const int64_t nyx = (int64_t)J.n[1] * J.n[2];
@@ -54,14 +62,22 @@ __device__ __forceinline__ bool query_voxel(const NectQueryJob &J, int64_t v, in
     const uint32_t in = (uint32_t)v & ((1u << ib) - 1u);
     const uint32_t nbx = ((uint32_t)J.n[2] + (1u << lx) - 1u) >> lx;
     const uint32_t nby = ((uint32_t)J.n[1] + (1u << ly) - 1u) >> ly;
+    const uint32_t nbz = ((uint32_t)J.n[0] + (1u << lz) - 1u) >> lz;
     const uint32_t plane = nby * nbx;
-    const uint32_t bz = b / plane;
-    const uint32_t r = b - bz * plane;
-    const uint32_t by = r / nbx;
-    const uint32_t bx = r - by * nbx;
-    iz = (int32_t)((bz << lz) + (in >> (ly + lx)));
-    iy = (int32_t)((by << ly) + ((in >> lx) & ((1u << ly) - 1u)));
-    ix = (int32_t)((bx << lx) + (in & ((1u << lx) - 1u)));
+    const uint32_t stack = min(32u >> lz, nbz);      // bricks per column of a layer (fewer in the last one)
+    const uint32_t layer = b / (stack * plane);
+    const uint32_t z0 = layer * stack;
+    if (z0 >= nbz) return false;                     // past the grid
+    const uint32_t tall = min(stack, nbz - z0);
+    const uint32_t r = b - z0 * plane;
+    const uint32_t col = r / tall;
+    const uint32_t at = ((r - col * tall) << ib) | in;
+    const uint32_t nz = tall << lz;
+    const uint32_t q = at / nz;
+    const uint32_t by = col / nbx;
+    iz = (int32_t)((z0 << lz) + (at - q * nz));
+    ix = (int32_t)(((col - by * nbx) << lx) + (q & ((1u << lx) - 1u)));
+    iy = (int32_t)((by << ly) + (q >> lx));
     return iz < J.n[0] && iy < J.n[1] && ix < J.n[2];
 }
 
@@ -73,11 +89,11 @@ __device__ __forceinline__ int64_t xcd_block(unsigned b, unsigned n) {
     return (int64_t)(b % kXcds) * (n / kXcds) + b / kXcds;
 }
 
-// The gathers are latency-bound: a register budget of three waves per SIMD
-// (the compiler fits it in ~125 VGPRs without spills, against ~190 unbounded)
-// lets three 4-wave workgroups share a CU, the most their LDS allows.
+// A register budget of four waves per SIMD (128 VGPRs; four 4-wave workgroups
+// share a CU, the most their LDS allows): the 512^3 query 29.0 ms, with three
+// 32.0.  Float32 images leave LDS for fewer.
 template <typename T, int D, int F>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_query(MlpArgs a, NectGridDesc g, const T *__restrict__ table,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 2 ? 4 : 3, 8))) void k_query(MlpArgs a, NectGridDesc g, const T *__restrict__ table,
                                                const NectQueryJob *__restrict__ jobs,
                                                const int64_t *__restrict__ prefix, int n_jobs, int64_t n_tiles,
                                                int out_f16, int x_stride) {
@@ -96,15 +112,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
         while (j + 1 < n_jobs && prefix[j + 1] <= tile) ++j;
         const NectQueryJob J = jobs[j];
         const int64_t first = (tile - prefix[j]) * kTile;
-        // output: lane s (both halves) holds voxel s of the tile
-        int32_t oz, oy, ox;
-        const bool rv = first + s < J.count && query_voxel(J, J.v0 + first + s, oz, oy, ox);
         // encoding: lanes 2e and 2e+1 gather the x-bit 0 and 1 corners of voxel e of the tile
+        bool rv;
+        int64_t out_at;
         {
             const int e = lane >> 1, cx = lane & 1;
             int32_t iz, iy, ix;
             const bool ev = first + e < J.count && query_voxel(J, J.v0 + first + e, iz, iy, ix);
             if (!ev) iz = iy = ix = 0;  // padding: any in-range voxel (never stored)
+            // output: lane s (both halves) stores voxel s of the tile
+            const int32_t oz = __shfl(iz, 2 * s), oy = __shfl(iy, 2 * s), ox = __shfl(ix, 2 * s);
+            rv = __shfl((int)ev, 2 * s) != 0;
+            out_at = ((int64_t)oz * J.n[1] + oy) * J.n[2] + ox;
             float p[D];
             p[0] = query_coord(J, 0, iz);
             p[1] = query_coord(J, 1, iy);
@@ -134,9 +153,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) voi
         const float zo = output_pre_last<T>(a, lds, 0, h, zl);
         const float y = rescale_value(J, act_fwd_slow(a.d.output_activation, zo));
         if (h == 0 && rv) {
-            const int64_t o = ((int64_t)oz * J.n[1] + oy) * J.n[2] + ox;
-            if (out_f16) static_cast<_Float16 *>(J.out)[o] = (_Float16)y;
-            else static_cast<float *>(J.out)[o] = y;
+            if (out_f16) static_cast<_Float16 *>(J.out)[out_at] = (_Float16)y;
+            else static_cast<float *>(J.out)[out_at] = y;
         }
         wave_lds_sync();
     }
