@@ -393,6 +393,38 @@ int32_t nect_calibrate_atomics(float *table, int64_t n_blocks, int32_t lanes_per
                                int64_t n_threads, uint32_t seed, void *stream);
 
 /*
+ * Table gradient through binned records, for batches large enough to stream
+ * (no reference counterpart: a schedule of the tiny-cuda-nn HashGrid backward).
+ * The same gradient as nect_grid_backward / nect_grid_backward_rays up to the
+ * order of float additions: every sample's contributions are first written as
+ * records sorted by the part of the table they fall into, then each part is
+ * summed on chip and added to grad once.
+ *
+ * The batch is taken in as many chunks as the workspace asks for.
+ * nect_grid_binned_workspace returns the bytes of a one-chunk workspace for
+ * n_slots samples (rays: 32 max_tiles), or of the largest one within max_bytes;
+ * 0 when the grid does not suit (a level of more than 2^24 (two features) or
+ * 2^23 (four) entries) or max_bytes is too small; negative on bad arguments.
+ * Any workspace (256-byte aligned) of at least the size returned for some
+ * max_bytes does.
+ *
+ * dout: rows of dout_stride elements of dout_dtype, each multiplied by
+ * *dout_scale (a device float) when dout_scale is set.  src_cols (rays): as in
+ * nect_grid_backward_ray_groups_cols; NULL for (z, y, x[, t]).
+ */
+int64_t nect_grid_binned_workspace(const NectGridDesc *desc, int64_t n_slots, int64_t max_bytes);
+
+int32_t nect_grid_backward_binned(const NectGridDesc *desc, const float *x, int64_t n, int64_t x_stride,
+                                  int32_t dout_dtype, const void *dout, int64_t dout_stride, const float *dout_scale,
+                                  float *grad, void *workspace, int64_t workspace_bytes, void *stream);
+
+int32_t nect_grid_backward_binned_rays(const NectGridDesc *desc, const int32_t *src_cols, const NectRay *rays,
+                                       const int32_t *tile_offsets, const int32_t *tile_ray, const int32_t *n_tiles,
+                                       int64_t max_tiles, float t, int32_t dout_dtype, const void *dout,
+                                       int64_t dout_stride, const float *dout_scale, float *grad, void *workspace,
+                                       int64_t workspace_bytes, void *stream);
+
+/*
  * Weight gradient of a wide network layer (tiny-cuda-nn's backward GEMM for
  * networks the fused kernels do not cover, configured at nect/config.py:125-132):
  * dw[i * ld_dw + j] += scale * sum over k < n_samples of dz[k * ld_dz + i] * h[k * ld_h + j]

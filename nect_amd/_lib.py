@@ -147,6 +147,10 @@ _SIGNATURES: dict[str, list] = {
     "nect_grid_backward_ray_groups_cols": [ctypes.POINTER(NectGridDesc), ctypes.POINTER(c_i32), c_vp, c_vp, c_i32,
                                            c_vp, c_i32, c_f32, c_i32, c_vp, c_i64, c_vp, c_vp,
                                            ctypes.POINTER(c_i32), c_i32, c_vp],
+    "nect_grid_backward_binned": [ctypes.POINTER(NectGridDesc), c_vp, c_i64, c_i64, c_i32, c_vp, c_i64, c_vp, c_vp, c_vp,
+                                  c_i64, c_vp],
+    "nect_grid_backward_binned_rays": [ctypes.POINTER(NectGridDesc), ctypes.POINTER(c_i32), c_vp, c_vp, c_vp, c_vp,
+                                       c_i64, c_f32, c_i32, c_vp, c_i64, c_vp, c_vp, c_vp, c_i64, c_vp],
     "nect_calibrate_atomics": [c_vp, c_i64, c_i32, c_i32, c_i64, ctypes.c_uint32, c_vp],
     "nect_wgrad": [c_i32, c_vp, c_i64, c_vp, c_i64, c_i64, c_i32, c_i32, c_f32, c_vp, c_i64, c_vp],
     "nect_gemm_act": [c_i32, c_vp, c_i64, c_vp, c_i64, c_i64, c_i32, c_i32, c_i32, c_f32, c_vp, c_i64, c_vp, c_i64,
@@ -166,6 +170,7 @@ _SIGNATURES: dict[str, list] = {
 _SIZE_QUERIES: dict[str, list] = {
     "nect_mlp_backward_workspace": [ctypes.POINTER(NectMlpDesc), c_i32, c_i64],
     "nect_ray_order_workspace": [ctypes.POINTER(NectGeometry)],
+    "nect_grid_binned_workspace": [ctypes.POINTER(NectGridDesc), c_i64, c_i64],
 }
 
 _lib: ctypes.CDLL | None = None

@@ -10,9 +10,8 @@ Replaces the body of BaseTrainer.fit's batch loop
     MLP          nect_mlp_forward                  mu [slots] (float)
     integral     nect_integral_loss                y_pred [B], loss, dmu [slots]
     backward     nect_mlp_backward                 dW (float), dfeat [slots, L*F]
-                 nect_ray_order +                  table gradient (float atomics over
-                 nect_grid_backward_ray_groups     groups of neighbouring rays, coarse
-                                                    levels summed per block in LDS)
+                 nect_grid_backward_binned_rays    table gradient (records sorted by table
+                                                    part, summed on chip)
     optimiser    nect_adam                         dense Adam + low-precision copy
 
 Every launch is asynchronous on torch's current stream; the step never
@@ -109,6 +108,54 @@ def loss_code(name: str) -> int:
     raise NotImplementedError(f"Loss {name} is not supported")
 
 
+class BinnedScatter:
+    """The record workspace of the binned table gradient (nect_grid_backward_binned*), kept between calls of one
+    owner (whose calls follow one another on one stream)."""
+
+    # Most bytes of records held at once; larger batches are taken in chunks, each adding its sums to the table once.
+    # Scatter of the 256^3 step (10.7 M samples) with 1.9 / 3.5 / 7 GiB: 6.4 / 6.1 / 5.9 ms; QuadCubes preset step
+    # (2^23-entry tables, whose sums cost most to add) with 6 / 12 / 24 GiB: 37.8 / 33.1 / 33.1 ms.
+    MAX_BYTES = 12 << 30
+    # Fewer samples than this, or than 1/2048 of the table's parameters, scatter straight to the table: the bins'
+    # sums are cleared and searched whatever the batch.  Direct / binned at 2^14, 2^15, 2^16 random points:
+    # 16 x 2 3-D, 2^19 entries 61 / 59, 118 / 77, 232 / 89 us; 19 x 4, 2^21 entries 100 / 128, 188 / 147, 376 / 223;
+    # 16 x 2 4-D, 2^21 entries 117 / 110, 229 / 165, 453 / 231.
+    MIN_SLOTS = 1 << 14
+
+    def __init__(self, device, max_bytes: int):
+        self.device = device
+        self.max_bytes = int(max_bytes)
+        self._buffer: torch.Tensor | None = None
+        self._sizes: dict = {}
+
+    def _need(self, grids, slots: int) -> int:
+        key = (slots, *[(g.n_dims, g.n_levels, g.n_features, g.n_params, g.struct.base_resolution) for g in grids])
+        need = self._sizes.get(key)
+        if need is None:
+            each = [int(_lib.lib().nect_grid_binned_workspace(g.struct_ref(), slots, self.max_bytes)) for g in grids]
+            need = max(each) if each and min(each) > 0 else 0
+            if len(self._sizes) > 64:
+                self._sizes.clear()
+            self._sizes[key] = need
+        return need
+
+    def suits(self, grids, slots: int) -> bool:
+        """Whether batches of ``slots`` samples take the binned schedule (every grid, one after another)."""
+        return (slots >= self.MIN_SLOTS and all(slots >= g.n_params >> 11 for g in grids)
+                and self._need(grids, slots) > 0)
+
+    def reserve(self, grids, slots: int):
+        need = self._need(grids, slots)
+        if self._buffer is None or self._buffer.numel() < need:
+            self._buffer = None   # the old one is returned before the new one is taken
+            self._buffer = torch.empty(need, dtype=torch.uint8, device=self.device)
+
+    def workspace(self, grids, slots: int) -> tuple[int, int]:
+        """(pointer, bytes) for a batch of ``slots`` samples."""
+        self.reserve(grids, slots)
+        return self._buffer.data_ptr(), self._buffer.numel()
+
+
 class FusedTrainStep:
     """Owns the parameters, Adam state and per-step buffers of one hash-grid model."""
 
@@ -117,7 +164,8 @@ class FusedTrainStep:
                  weight_decay: float = 0.0, memory_budget: int | None = None):
         """``memory_budget`` (bytes) bounds the per-sample buffers (features, their gradients, mu, dmu): a batch
         whose samples exceed it is processed in chunks of rays that fit, each chunk's gradient weighted by its
-        share of the batch, and one optimiser step at the end."""
+        share of the batch, and one optimiser step at the end.  It also bounds the table gradient's record
+        workspace, which is a buffer of its own."""
         if mlp.n_input != grid.n_output_dims:
             raise ValueError("MLP input width must equal the grid's L*F")
         if params.dtype != torch.float32 or not params.is_cuda:
@@ -157,16 +205,19 @@ class FusedTrainStep:
         # writes whole rows of its own plane); the MLP reads that layout directly
         self.grouped = grid.n_levels % 8 == 0 and mlp.n_input == mlp.n_input_padded
         self.memory_budget = memory_budget
-        # table-gradient schedule: "groups" (nect_ray_order + nect_grid_backward_ray_groups) or "tiles"
-        # (nect_grid_backward_rays in batch order); n_agg_levels None picks aggregated_levels()
-        self.scatter = "groups"
-        # the grouped schedule's patch order applied to the whole step (see _presort)
+        # table-gradient schedule: "bins" (nect_grid_backward_binned_rays), "groups" (nect_ray_order +
+        # nect_grid_backward_ray_groups) or "tiles" (nect_grid_backward_rays in batch order); batches that "bins"
+        # does not suit (see _use_bins) take "groups" or "tiles" by size
+        self.scatter = "bins"
+        # large batches are taken in detector-patch order for the whole step (see _presort)
         self.presort = True
         self._y_sorted = torch.empty(0, dtype=torch.float32, device=self.device)
         self.agg_rounds: list[int] | None = None   # per level; None: aggregation_plan()
         self.scatter_split = False
         self._order_ws = torch.empty(0, dtype=torch.uint8, device=self.device)
         self._order_need: dict = {}
+        self._bins = BinnedScatter(self.device, BinnedScatter.MAX_BYTES if memory_budget is None
+                                   else min(BinnedScatter.MAX_BYTES, memory_budget))
         self._plan_cache: dict = {}
         self._chunk_counts: list = []
         self._alloc(max_rays, max_points_per_ray)
@@ -233,6 +284,8 @@ class FusedTrainStep:
         self.loss_value = torch.empty(1, dtype=torch.float32, device=dev)
         ws = int(_lib.lib().nect_mlp_backward_workspace(self.mlp.struct_ref(), _lib.dtype_code(self.dtype), slots))
         self.workspace = torch.empty(max(ws, 16), dtype=torch.uint8, device=dev)
+        if self._use_bins(slots):
+            self._bins.reserve([self.grid], slots)
 
     @property
     def mlp_weights(self) -> torch.Tensor:
@@ -322,15 +375,15 @@ class FusedTrainStep:
                    _lib.ptr(self.mlp_weights), _lib.ptr(self.features), slots, F, self._x_groups(),
                    _lib.ptr(self.n_tiles), _lib.ptr(self.dmu), 1, loss_scale, loss_scale_dev, float(share),
                    _lib.ptr(self.grad), _lib.ptr(self.dfeat), F, _lib.ptr(self.workspace), self.workspace.numel(), st)
-        if perm is None:
+        if perm is None and self._use_groups(num_rays, points_per_ray):
             self._ray_order(geometry, ray_index, start, num_rays, points_per_ray)
         self._grid_backward(geometry, num_rays, points_per_ray, step_mm, max_tiles, t, ordered=perm is None)
 
     def _presort(self, geometry, ray_index, start: int, num_rays: int, points_per_ray: int):
-        """With ``presort`` and the grouped schedule: the patch order of the batch (int64), which the whole step
+        """With ``presort``, for large batches: the patch order of the batch (int64), which the whole step
         then follows -- the encoder's gathers of neighbouring rays share L2 lines, the scatter's groups are
         consecutive rays; per-ray outputs are returned in the caller's order.  None otherwise."""
-        if not (self.presort and self._use_groups(num_rays, points_per_ray)):
+        if not (self.presort and self._many(num_rays, points_per_ray)):
             return None
         self._ray_order(geometry, ray_index, start, num_rays, points_per_ray)
         if self._y_sorted.numel() < num_rays:
@@ -355,13 +408,19 @@ class FusedTrainStep:
     # leave the device idle, and the tile schedule (one wave per 32 samples) is faster
     GROUPS_MIN_WORKGROUPS = 2048
 
-    def _use_groups(self, num_rays: int, points_per_ray: int) -> bool:
+    def _many(self, num_rays: int, points_per_ray: int) -> bool:
         passes = 2 * ((points_per_ray + 31) // 32)
-        return self.scatter == "groups" and ((num_rays + 63) // 64) * passes >= self.GROUPS_MIN_WORKGROUPS
+        return self.scatter != "tiles" and ((num_rays + 63) // 64) * passes >= self.GROUPS_MIN_WORKGROUPS
+
+    def _use_bins(self, slots: int) -> bool:
+        return self.scatter == "bins" and self._bins.suits([self.grid], slots)
+
+    def _use_groups(self, num_rays: int, points_per_ray: int) -> bool:
+        return self._many(num_rays, points_per_ray) and not self._use_bins(cs.tiles_needed(num_rays, points_per_ray) * 32)
 
     def _ray_order(self, geometry, ray_index: torch.Tensor, start: int, num_rays: int, points_per_ray: int):
         """Groups the batch's rays by detector patch for the grouped scatter (self.order)."""
-        if not self._use_groups(num_rays, points_per_ray):
+        if not self._many(num_rays, points_per_ray):
             return
         g = geometry._struct()
         key = tuple(geometry.nDetector)
@@ -402,7 +461,12 @@ class FusedTrainStep:
         F = self.grid.n_output_dims
         rays = self.rays[:num_rays]
         grad = self.grad[self.n_mlp:].data_ptr()
-        if self._use_groups(num_rays, points_per_ray):
+        if self._use_bins(max_tiles * 32):
+            ws, ws_bytes = self._bins.workspace([self.grid], max_tiles * 32)
+            self._call("grid_backward", "nect_grid_backward_binned_rays", self.grid.struct_ref(), None, _lib.ptr(rays),
+                       _lib.ptr(self.tile_offsets), _lib.ptr(self.tile_ray), _lib.ptr(self.n_tiles), int(max_tiles),
+                       float(t), _lib.F32, _lib.ptr(self.dfeat), F, None, grad, ws, ws_bytes, st)
+        elif self._use_groups(num_rays, points_per_ray):
             self._call("grid_backward", "nect_grid_backward_ray_groups", self.grid.struct_ref(), _lib.ptr(rays),
                        _lib.ptr(self.tile_offsets), int(num_rays), _lib.ptr(self.order) if ordered else None,
                        int(points_per_ray), float(t), _lib.ptr(self.dfeat), F, grad,
@@ -463,7 +527,7 @@ class FusedTrainStep:
             gy = torch.sign(diff) / num_rays
         gy = gy.contiguous()
         F = self.grid.n_output_dims
-        if perm is None:
+        if perm is None and self._use_groups(num_rays, points_per_ray):
             self._ray_order(geometry, ray_index, starting_ray_index, num_rays, points_per_ray)
         for k in range(K):
             max_tiles = self.forward_rays(geometry, angles[k], ray_index, starting_ray_index, num_rays,

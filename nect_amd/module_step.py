@@ -20,9 +20,10 @@ modules scale the backward by a power of two of max |dL/dy| themselves.
 
 Large batches of a model that names its grids' sample coordinates (``grid_sources``) follow the fused path's
 schedule: the batch is taken in detector-patch order (nect_ray_order), so neighbouring rays' samples are
-encoded together, and each grid's table gradient is scattered over groups of 64 neighbouring rays with the
-coarse levels summed in LDS (nect_grid_backward_ray_groups_cols), replacing the module's per-sample scatter;
-line integrals are returned in the caller's order.
+encoded together, and each grid's table gradient goes through binned records (nect_grid_backward_binned_rays;
+grids that does not suit: over groups of 64 neighbouring rays with the coarse levels summed in LDS,
+nect_grid_backward_ray_groups_cols), replacing the module's per-sample scatter; line integrals are returned in
+the caller's order.
 """
 from __future__ import annotations
 
@@ -31,7 +32,7 @@ import ctypes
 import torch
 
 from . import _lib
-from .fused import LOSS_GIVEN, aggregation_plan, loss_code
+from .fused import LOSS_GIVEN, BinnedScatter, aggregation_plan, loss_code
 from .sampling import ct_sampling as cs
 
 
@@ -63,8 +64,10 @@ class ModuleTrainStep:
         if self.amp:
             _lib.call("nect_amp_init", _lib.ptr(self.amp_state), 1.0, _lib.stream_of(self.device))
         self.amp_growth_interval = 2000
-        # table-gradient schedule: "groups" (ray groups, patch order) when the model names its grids' coordinates
-        self.scatter = "groups" if getattr(model, "grid_sources", None) is not None else "module"
+        # table-gradient schedule when the model names its grids' coordinates: "bins" (records sorted by table part)
+        # or "groups" (ray groups); "module" leaves it to the module's own backward
+        self.scatter = "bins" if getattr(model, "grid_sources", None) is not None else "module"
+        self._bins = BinnedScatter(self.device, BinnedScatter.MAX_BYTES)
         self.presort = True
         self.agg_rounds: list | None = None      # per grid, per level; None: aggregation_plan()
         # the scatter's launches (nect_grid_backward_ray_groups' split): 0 one launch per grid, 1 the aggregated
@@ -154,7 +157,13 @@ class ModuleTrainStep:
 
     def _use_groups(self, num_rays: int, points_per_ray: int) -> bool:
         passes = 2 * ((points_per_ray + 31) // 32)
-        return self.scatter == "groups" and ((num_rays + 63) // 64) * passes >= self.GROUPS_MIN_WORKGROUPS
+        return self.scatter != "module" and ((num_rays + 63) // 64) * passes >= self.GROUPS_MIN_WORKGROUPS
+
+    def _grids(self):
+        return [p.desc for p in self.model.net.grid_parts()]
+
+    def _use_bins(self, slots: int) -> bool:
+        return self.scatter == "bins" and self._bins.suits(self._grids(), slots)
 
     def _ray_order(self, geometry, ray_index: torch.Tensor, start: int, num_rays: int):
         """self.order: the batch's rays grouped by 8x8 detector patch (nect_ray_order)."""
@@ -201,8 +210,7 @@ class ModuleTrainStep:
     def _grid_scatter(self, geometry, num_rays: int, points_per_ray: int, step_mm: float, t: float, ordered: bool,
                       dfeat: torch.Tensor, grad: torch.Tensor, dfeat_scale: torch.Tensor | None = None):
         """Each grid's table gradient from dL/dfeatures [slots, n_encoded] (= dfeat * dfeat_scale when the scale
-        is given: the network's 16-bit loss-scaled result, unscaled as the scatter reads it) over the batch's ray
-        groups."""
+        is given: the network's 16-bit loss-scaled result, unscaled as the scatter reads it)."""
         st = _lib.stream_of(self.device)
         rays = self.rays[:num_rays]
         if dfeat.stride(1) != 1:
@@ -211,6 +219,16 @@ class ModuleTrainStep:
             dfeat_scale = dfeat_scale.float().contiguous()
         n_enc = dfeat.stride(0)
         esz = dfeat.element_size()
+        max_tiles = cs.tiles_needed(num_rays, points_per_ray)
+        if self._use_bins(max_tiles * 32):
+            ws, ws_bytes = self._bins.workspace(self._grids(), max_tiles * 32)
+            for part, src in zip(self.model.net.grid_parts(), self.model.grid_sources):
+                cols = (ctypes.c_int32 * len(src))(*src)
+                _lib.call("nect_grid_backward_binned_rays", part.desc.struct_ref(), cols, _lib.ptr(rays),
+                          _lib.ptr(self.tile_offsets), _lib.ptr(self.tile_ray), _lib.ptr(self.n_tiles), int(max_tiles),
+                          float(t), _lib.dtype_code(dfeat.dtype), dfeat.data_ptr() + esz * part.out0, n_enc,
+                          _lib.ptr(dfeat_scale), grad.data_ptr() + 4 * part.p0, ws, ws_bytes, st)
+            return
         for k, (part, src) in enumerate(zip(self.model.net.grid_parts(), self.model.grid_sources)):
             cols = (ctypes.c_int32 * len(src))(*src)
             _lib.call("nect_grid_backward_ray_groups_cols", part.desc.struct_ref(), cols, _lib.ptr(rays),
@@ -256,7 +274,7 @@ class ModuleTrainStep:
         self._integral(num_rays, mu.detach(), target.contiguous(), l_max, self.loss, y_buf)
         if perm is not None:
             self.y_pred[:num_rays].index_copy_(0, perm, y_buf[:num_rays])
-        elif groups:
+        elif groups and not self._use_bins(slots):
             self._ray_order(geometry, ray_index, starting_ray_index, num_rays)
         self._zero_grad()
         self._backward(mu, slots, geometry, num_rays, points_per_ray, step_mm, t, groups, ordered=perm is None)
@@ -294,7 +312,7 @@ class ModuleTrainStep:
         gy = (gy / K).contiguous()
         self._zero_grad()
         groups = self._use_groups(num_rays, points_per_ray)
-        if groups:
+        if groups and not self._use_bins(cs.tiles_needed(num_rays, points_per_ray) * 32):
             self._ray_order(geometry, ray_index, starting_ray_index, num_rays)   # the same pixels at every sub-angle
         for k in range(K):
             slots = self._positions(geometry, angles[k], ray_index, starting_ray_index, num_rays, points_per_ray,

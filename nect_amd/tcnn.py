@@ -31,9 +31,11 @@ import torch.nn.functional as F
 from . import _lib
 from . import grid as _grid
 from . import mlp as _mlp
-from .fused import xavier_init
+from .fused import BinnedScatter, xavier_init
 
 MAX_GRID_PARTS = 5   # NECT_MAX_GRID_PARTS
+# most bytes of records the table gradient of a caller's points takes from torch's allocator for a backward
+POINTS_SCATTER_BYTES = 2 << 30
 
 
 def torch_activation(name: str | None, z: torch.Tensor) -> torch.Tensor:
@@ -183,6 +185,16 @@ def _encode_backward(parts: list[_Part], x: torch.Tensor, dfeat: torch.Tensor, g
         return
     if dfeat.stride(1) != 1:
         dfeat = dfeat.contiguous()
+    if x.shape[0] >= BinnedScatter.MIN_SLOTS:
+        grids = [p for p in parts if p.kind == "grid"]
+        bins = BinnedScatter(x.device, POINTS_SCATTER_BYTES)
+        if grids and bins.suits([p.desc for p in grids], x.shape[0]):
+            ws, ws_bytes = bins.workspace([p.desc for p in grids], x.shape[0])
+            for p in grids:
+                _lib.call("nect_grid_backward_binned", p.desc.struct_ref(), _lib.ptr(x) + 4 * p.col0, x.shape[0],
+                          x.shape[1], _lib.F32, dfeat.data_ptr() + 4 * p.out0, dfeat.stride(0), None,
+                          _lib.ptr(grad) + 4 * p.p0, ws, ws_bytes, _lib.stream_of(x.device))
+            return
     for group in _launch_groups(parts):
         n, descs, offs, cols, outs = _parts_args(group)
         _lib.call("nect_grid_backward_parts", n, descs, offs, cols, outs, _lib.ptr(x), x.shape[0], x.shape[1],
