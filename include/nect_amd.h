@@ -132,6 +132,15 @@ int32_t nect_ray_tiles(const NectRay *rays, int32_t num_rays, int64_t max_tiles,
  * random order, projector.py:93-130); it only schedules work.
  */
 int64_t nect_ray_order_workspace(const NectGeometry *geometry);
+
+/* The same along detector columns: patches of 64 rows x 1 column, column by
+ * column, their rays by row, so that consecutive rays are neighbours along the
+ * columns (for a detector whose columns follow the rotation axis: along z). */
+int64_t nect_ray_order_columns_workspace(const NectGeometry *geometry);
+int32_t nect_ray_order_columns(const NectGeometry *geometry, const int64_t *ray_index, int64_t n_ray_index,
+                               int32_t num_rays, int32_t starting_ray_index, int32_t *order, void *workspace,
+                               int64_t workspace_bytes, void *stream);
+
 int32_t nect_ray_order(const NectGeometry *geometry, const int64_t *ray_index, int64_t n_ray_index,
                        int32_t num_rays, int32_t starting_ray_index, int32_t *order, void *workspace,
                        int64_t workspace_bytes, void *stream);
@@ -327,6 +336,16 @@ int32_t nect_grid_encode_rays(const NectGridDesc *desc, int32_t dtype, const voi
                               const int32_t *tile_offsets, const int32_t *tile_ray, const int32_t *n_tiles,
                               int64_t max_tiles, float t, void *out, int64_t out_stride, int32_t grouped,
                               void *stream);
+
+/* The features nect_grid_encode_rays writes, bit for bit, by another schedule:
+ * a wave encodes one sample of 32 consecutive rays at a time, which gathers from
+ * few cache lines when the rays are ordered along detector columns
+ * (nect_ray_order_columns).  Any order of the rays is correct.  Slots of the
+ * rays' tiles only are written; out must be aligned to one level's features. */
+int32_t nect_grid_encode_ray_columns(const NectGridDesc *desc, int32_t dtype, const void *table, const NectRay *rays,
+                                     const int32_t *tile_offsets, int32_t num_rays, int32_t max_points_per_ray,
+                                     int64_t max_tiles, float t, void *out, int64_t out_stride, int32_t grouped,
+                                     void *stream);
 
 /* nect_grid_backward over the samples of the fused path (dout float,
  * [max_tiles*32, L*F], row stride dout_stride). */

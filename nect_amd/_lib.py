@@ -121,6 +121,7 @@ _SIGNATURES: dict[str, list] = {
                        c_vp, c_vp, c_vp, c_vp],
     "nect_ray_tiles": [c_vp, c_i32, c_i64, c_vp, c_vp, c_vp, c_vp],
     "nect_ray_positions": [c_vp, c_vp, c_vp, c_vp, c_i64, c_vp, c_vp, c_vp],
+    "nect_ray_order_columns": [ctypes.POINTER(NectGeometry), c_vp, c_i64, c_i32, c_i32, c_vp, c_vp, c_i64, c_vp],
     "nect_ray_order": [ctypes.POINTER(NectGeometry), c_vp, c_i64, c_i32, c_i32, c_vp, c_vp, c_i64, c_vp],
     "nect_grid_init": [ctypes.POINTER(NectGridDesc), c_i32, c_i32, c_i32, c_i32, c_i32, c_f32],
     "nect_grid_index": [ctypes.POINTER(NectGridDesc), c_vp, c_i64, c_i64, c_vp, c_vp, c_vp],
@@ -138,6 +139,8 @@ _SIGNATURES: dict[str, list] = {
     "nect_mlp_backward_noalloc": [ctypes.POINTER(NectMlpDesc), c_i32, c_vp, c_vp, c_i64, c_i64,
                                   ctypes.POINTER(NectGridDesc), c_vp, c_vp, c_i64, c_f32, c_vp, c_f32, c_vp, c_vp, c_i64,
                                   c_vp],
+    "nect_grid_encode_ray_columns": [ctypes.POINTER(NectGridDesc), c_i32, c_vp, c_vp, c_vp, c_i32, c_i32, c_i64, c_f32,
+                                     c_vp, c_i64, c_i32, c_vp],
     "nect_grid_encode_rays": [ctypes.POINTER(NectGridDesc), c_i32, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_f32, c_vp,
                               c_i64, c_i32, c_vp],
     "nect_grid_backward_rays": [ctypes.POINTER(NectGridDesc), c_vp, c_vp, c_vp, c_vp, c_i64, c_f32, c_vp, c_i64, c_vp,
@@ -170,6 +173,7 @@ _SIGNATURES: dict[str, list] = {
 _SIZE_QUERIES: dict[str, list] = {
     "nect_mlp_backward_workspace": [ctypes.POINTER(NectMlpDesc), c_i32, c_i64],
     "nect_ray_order_workspace": [ctypes.POINTER(NectGeometry)],
+    "nect_ray_order_columns_workspace": [ctypes.POINTER(NectGeometry)],
     "nect_grid_binned_workspace": [ctypes.POINTER(NectGridDesc), c_i64, c_i64],
 }
 

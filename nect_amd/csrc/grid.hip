@@ -143,6 +143,122 @@ __global__ __launch_bounds__(256) void k_grid_encode_pair(NectGridDesc g, const 
     encode_pair_tile<D, F, T, Src, GROUPED>(g, table, src, n_slots, out, out_stride, n_groups, vpp, blockIdx.x);
 }
 
+// Encoder over ray groups: a wave takes 32 consecutive rays and one tile index,
+// and encodes one sample index of all of them at a time (lane pair e: ray e), so
+// that with rays ordered along detector columns an instruction's samples lie
+// along z.  z is the grid's first coordinate, whose neighbouring cells are
+// neighbouring table entries on dense and hashed levels alike: the gathers, bound
+// by the cache lines an instruction touches, then touch a fraction of those that
+// 32 samples along one ray do.  Encoder of one step, k_grid_encode_pair in patch
+// order -> this kernel in column order: 262144 x 256 samples, 16 levels, FP16
+// 3.04 -> 1.62 ms; 4-D BF16 7.73 -> 5.76; 20 levels of 4 features 1.06 -> 0.65;
+// FP32 0.83 -> 0.50; below about 8192 rays of 128 samples the other way round
+// (1024 x 64: 0.021 -> 0.050 ms, too few waves in flight).
+// PLANAR: the level-grouped schedule and planes of k_grid_encode_pair; else one
+// group of all levels and rows of out_stride elements.  The features of CH
+// samples of the wave's rays are assembled in LDS and written back as whole
+// stretches of a ray (the slots of a tile follow one another).
+template <int D, int F, typename T, bool PLANAR>
+__global__ __launch_bounds__(256) void k_grid_encode_columns(NectGridDesc g, const T *__restrict__ table,
+                                                             const NectRay *__restrict__ rays,
+                                                             const int32_t *__restrict__ tile_offsets, int num_rays,
+                                                             int n_passes, float t, T *__restrict__ out,
+                                                             int64_t out_stride, int n_groups, int64_t n_slots,
+                                                             int width, int ch, int vec) {
+    extern __shared__ __align__(16) char smem_raw[];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const int e = lane >> 1, cx = lane & 1;
+    const int grp = PLANAR ? (int)(blockIdx.x % (unsigned)n_groups) : 0;
+    const unsigned block = PLANAR ? blockIdx.x / (unsigned)n_groups : blockIdx.x;
+    const unsigned unit = block * 4 + wave;
+    const unsigned rg = unit / (unsigned)n_passes;
+    const int j = (int)(unit - rg * (unsigned)n_passes);
+    // a ray's ch samples of `width` elements, and 16 bytes so that the lanes' rows start on different banks
+    const int row = ch * width + 16 / (int)sizeof(T);
+    T *stage = reinterpret_cast<T *>(smem_raw) + wave * kTile * row;
+    const int r = (int)rg * kTile + e;
+    int64_t slot0 = -1;   // first slot of the ray's tile j
+    NectRay d;
+    d.count = 0;
+    if (r < num_rays) {
+        const int32_t a = tile_offsets[r];
+        if (j < tile_offsets[r + 1] - a && (int64_t)(a + j) * kTile < n_slots) {
+            slot0 = (int64_t)(a + j) * kTile;
+            d = rays[r];
+        }
+    }
+    if (__ballot(slot0 >= 0) == 0) return;
+    for (int i0 = 0; i0 < kTile; i0 += ch) {
+        for (int i = i0; i < i0 + ch; ++i) {
+            float q[3] = {0.0f, 0.0f, 0.0f};
+            const bool ok = slot0 >= 0 && ray_sample(d, kTile * j + i, q);
+            T *o = stage + e * row + (i - i0) * width;
+            if (__ballot(ok) == 0) {
+                for (int c = cx; c < width; c += 2) o[c] = from_f32<T>(0.0f);
+                continue;
+            }
+            float p[D];
+#pragma unroll
+            for (int k = 0; k < D && k < 3; ++k) p[k] = ok ? q[k] : 0.0f;
+            if (D == 4) p[D - 1] = t;
+            for (int jl = 0;; ++jl) {
+                const int l = PLANAR ? group_level(grp, jl, n_groups) : jl;
+                if (l >= g.n_levels) break;
+                const LevelInfo lv = level_info(g, l);
+                uint32_t c[D];
+                float f[D];
+#pragma unroll
+                for (int k = 0; k < D; ++k) grid_pos(lv.scale, p[k], c[k], f[k]);
+                float v[F];
+                encode_half<D, F, T>(lv, c, f, table, cx, v);
+                float sum[F];
+#pragma unroll
+                for (int k = 0; k < F; ++k) {
+                    const float other = __shfl_xor(v[k], 1, kWave);
+                    sum[k] = cx == 0 ? v[k] + other : other + v[k];
+                }
+                if (cx == (l & 1)) {
+#pragma unroll
+                    for (int k = 0; k < F; ++k) o[jl * F + k] = from_f32<T>(ok ? sum[k] : 0.0f);
+                }
+            }
+        }
+        // the wave's own LDS rows: LDS operations of one wave complete in order
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+        // whole waves stay in the loops: slot0 is read from other lanes
+        if (vec) {
+            // a ray's samples are one stretch of memory: 16 bytes per lane
+            constexpr int V = 16 / (int)sizeof(T);
+            const int per_ray = ch * width / V;
+            T *dst0 = out + (PLANAR ? (int64_t)grp * n_slots * width : 0) + (int64_t)i0 * width;
+            for (int k0 = 0; k0 < kTile * per_ray; k0 += kWave) {
+                const int er = min((k0 + lane) / per_ray, kTile - 1), w = k0 + lane - er * per_ray;
+                const int64_t s0 = __shfl(slot0, 2 * er, kWave);
+                if (s0 >= 0 && w < per_ray)
+                    *reinterpret_cast<uint4 *>(dst0 + s0 * width + w * V) =
+                        *reinterpret_cast<const uint4 *>(stage + er * row + w * V);
+            }
+        } else {
+            using Chunk = typename ChunkOf<F * (int)sizeof(T)>::type;
+            const int pieces = width / F, per_ray = ch * pieces;   // a sample's features in pieces of F
+            for (int k0 = 0; k0 < kTile * per_ray; k0 += kWave) {
+                const int er = min((k0 + lane) / per_ray, kTile - 1), w = k0 + lane - er * per_ray;
+                const int i = w / pieces, c = (w - i * pieces) * F;
+                const int64_t s0 = __shfl(slot0, 2 * er, kWave);
+                if (s0 < 0 || w >= per_ray) continue;
+                T *dst = PLANAR ? out + (int64_t)grp * n_slots * width + (s0 + i0 + i) * width + c
+                                : out + (s0 + i0 + i) * out_stride + c;
+                *reinterpret_cast<Chunk *>(dst) = *reinterpret_cast<const Chunk *>(stage + er * row + i * width + c);
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+    }
+}
+
 // Sum of v over samples m..end of this lane's pass (lanes 4m..4m+3 hold sample m);
 // complete at the run's first sample.
 __device__ __forceinline__ float run_sum_quad(float v, int m, int end) {
@@ -756,6 +872,49 @@ static int32_t launch_encode(const NectGridDesc &g, int32_t dtype, const void *t
     return check_launch("k_grid_encode_pair");
 }
 
+static int32_t launch_encode_columns(const NectGridDesc &g, int32_t dtype, const void *table, const NectRay *rays,
+                                     const int32_t *tile_offsets, int num_rays, int n_passes, float t, void *out,
+                                     int64_t out_stride, bool planar, int64_t n_slots, hipStream_t st) {
+    const int G = planar ? 8 : 1;
+    const int esz = dtype == NECT_F32 ? 4 : 2;
+    const int width = planar ? grouped_vpp(g) : g.n_levels * g.n_features;
+    // samples assembled at once (16 of them: 256^3 step's encoder 1.62 ms, 32: 1.73, fewer workgroups fit a CU; with
+    // 8 the float32 one 0.57 ms, with 16 0.50), up to 9 KiB per wave
+    int ch = 16;
+    while (ch > 1 && (size_t)kTile * (ch * width * esz + 16) > 9 * 1024) ch /= 2;
+    const size_t lds = (size_t)4 * kTile * (ch * width * esz + 16);
+    const int vec = (planar || out_stride == width) && ch * width * esz % 16 == 0 && (uintptr_t)out % 16 == 0 &&
+                    n_slots * width * esz % 16 == 0;
+    const int64_t units = (int64_t)((num_rays + kTile - 1) / kTile) * n_passes;
+    NECT_REQUIRE((units + 3) / 4 * G < ((int64_t)1 << 31), "too many ray groups");
+    const dim3 grid((unsigned)((units + 3) / 4 * G)), block(256);
+#define NECT_ENCC(D, F, T, P)                                                                                       \
+    hipLaunchKernelGGL((k_grid_encode_columns<D, F, T, P>), grid, block, lds, st, g, (const T *)table, rays,         \
+                       tile_offsets, num_rays, n_passes, t, (T *)out, out_stride, G, n_slots, width, ch, vec)
+#define NECT_ENCC_P(D, F, T)                       \
+    do {                                           \
+        if (planar) NECT_ENCC(D, F, T, true);      \
+        else NECT_ENCC(D, F, T, false);            \
+    } while (0)
+#define NECT_ENCC_T(D, F)                                  \
+    do {                                                   \
+        if (dtype == NECT_F32) NECT_ENCC_P(D, F, float);   \
+        else if (dtype == NECT_F16) NECT_ENCC_P(D, F, _Float16); \
+        else NECT_ENCC_P(D, F, bf16_t);                    \
+    } while (0)
+    if (g.n_dims == 3) {
+        if (g.n_features == 2) NECT_ENCC_T(3, 2);
+        else NECT_ENCC_T(3, 4);
+    } else {
+        if (g.n_features == 2) NECT_ENCC_T(4, 2);
+        else NECT_ENCC_T(4, 4);
+    }
+#undef NECT_ENCC_T
+#undef NECT_ENCC_P
+#undef NECT_ENCC
+    return check_launch("k_grid_encode_columns");
+}
+
 template <typename Src3, typename Src4>
 static int32_t launch_backward(const NectGridDesc &g, const Src3 &s3, const Src4 &s4, int64_t n_slots,
                                const float *dout, int64_t dout_stride, float *grad, hipStream_t st) {
@@ -939,6 +1098,30 @@ extern "C" int32_t nect_grid_encode_rays(const NectGridDesc *desc, int32_t dtype
     RaySource<3> s3{rays, tile_offsets, tile_ray, n_tiles, t};
     RaySource<4> s4{rays, tile_offsets, tile_ray, n_tiles, t};
     return launch_encode(*desc, dtype, table, s3, s4, max_tiles * kTile, out, out_stride, vpp, as_stream(stream));
+}
+
+extern "C" int32_t nect_grid_encode_ray_columns(const NectGridDesc *desc, int32_t dtype, const void *table,
+                                                const NectRay *rays, const int32_t *tile_offsets, int32_t num_rays,
+                                                int32_t max_points_per_ray, int64_t max_tiles, float t, void *out,
+                                                int64_t out_stride, int32_t grouped, void *stream) {
+    clear_error();
+    if (check_grid(desc)) return 1;
+    NECT_REQUIRE(dtype >= NECT_F32 && dtype <= NECT_BF16, "unknown dtype");
+    NECT_REQUIRE(num_rays >= 0 && max_points_per_ray >= 1, "num_rays must be >= 0 and max_points_per_ray >= 1");
+    if (num_rays == 0) return 0;
+    NECT_REQUIRE(table && rays && tile_offsets && out, "NULL pointer");
+    NECT_REQUIRE(max_tiles >= 1, "max_tiles must be >= 1");
+    const int64_t piece = desc->n_features * (dtype == NECT_F32 ? 4 : 2);
+    if (grouped) {
+        NECT_REQUIRE(desc->n_levels % 8 == 0, "the grouped feature layout needs a multiple of 8 levels");
+    } else {
+        NECT_REQUIRE(out_stride >= (int64_t)desc->n_levels * desc->n_features, "out_stride smaller than L*F");
+        NECT_REQUIRE(out_stride % desc->n_features == 0, "out_stride must be a multiple of n_features_per_level");
+    }
+    NECT_REQUIRE((uintptr_t)out % piece == 0, "out must be aligned to one level's features");
+    return launch_encode_columns(*desc, dtype, table, rays, tile_offsets, num_rays,
+                                 (max_points_per_ray + kTile - 1) / kTile, t, out, out_stride, grouped != 0,
+                                 max_tiles * kTile, as_stream(stream));
 }
 
 extern "C" int32_t nect_grid_backward_rays(const NectGridDesc *desc, const NectRay *rays,

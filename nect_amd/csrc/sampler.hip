@@ -225,8 +225,11 @@ __global__ __launch_bounds__(256) void k_ray_positions(const NectRay *__restrict
 // A patch that holds a pixel twice keeps an arbitrary order.
 constexpr int kPatch = 8;
 
+// tall: patches of 64 rows x 1 column (numbered column by column), their rays
+// from the first row to the last, for kernels that take neighbours along z.
 struct PatchKey {
-    int cols, pcols, n_cells;  // detector columns, patch columns, patches
+    int cols, pcols, n_cells;  // detector columns, patches per row of patches (tall: per column), patches
+    int tall;                  // the detector's rows, or 0
     // patch of ray t (n_cells: no pixel) and its position in the patch (0..63)
     __device__ __forceinline__ int of(const int64_t *ray_index, int64_t n_ray_index, int start, int t,
                                       int &pos) const {
@@ -235,6 +238,11 @@ struct PatchKey {
         const int64_t pix = ray_index[t + start];
         if (pix < 0) return n_cells;
         const int64_t row = pix / cols, col = pix % cols;
+        if (tall) {
+            if (row >= tall) return n_cells;
+            pos = (int)(row % 64);
+            return (int)(col * pcols + row / 64);
+        }
         const int64_t key = (row / kPatch) * pcols + col / kPatch;
         if (key >= n_cells) return n_cells;
         const int r = (int)(row % kPatch), c = (int)(col % kPatch);
@@ -320,8 +328,15 @@ __global__ __launch_bounds__(256) void k_order_place(PatchKey pk, const int64_t 
     order[slot] = t;
 }
 
-static PatchKey patch_key(const NectGeometry &g) {
+static PatchKey patch_key(const NectGeometry &g, bool tall = false) {
     PatchKey pk;
+    pk.tall = tall ? g.n_det[0] : 0;
+    if (tall) {
+        pk.cols = g.n_det[1];
+        pk.pcols = (g.n_det[0] + 63) / 64;
+        pk.n_cells = pk.pcols * g.n_det[1];
+        return pk;
+    }
     pk.cols = g.n_det[1];
     pk.pcols = (g.n_det[1] + kPatch - 1) / kPatch;
     pk.n_cells = pk.pcols * ((g.n_det[0] + kPatch - 1) / kPatch);
@@ -429,16 +444,41 @@ extern "C" int64_t nect_ray_order_workspace(const NectGeometry *geometry) {
     return 20 * ((int64_t)patch_key(*geometry).n_cells + 1);
 }
 
+extern "C" int64_t nect_ray_order_columns_workspace(const NectGeometry *geometry) {
+    clear_error();
+    if (check_geometry(geometry)) return -1;
+    return 20 * ((int64_t)patch_key(*geometry, true).n_cells + 1);
+}
+
+static int32_t order_rays(const PatchKey &pk, const int64_t *ray_index, int64_t n_ray_index, int32_t num_rays,
+                          int32_t starting_ray_index, int32_t *order, void *workspace, int64_t workspace_bytes,
+                          void *stream);
+
+extern "C" int32_t nect_ray_order_columns(const NectGeometry *geometry, const int64_t *ray_index, int64_t n_ray_index,
+                                          int32_t num_rays, int32_t starting_ray_index, int32_t *order,
+                                          void *workspace, int64_t workspace_bytes, void *stream) {
+    clear_error();
+    if (check_geometry(geometry)) return 1;
+    return order_rays(patch_key(*geometry, true), ray_index, n_ray_index, num_rays, starting_ray_index, order,
+                      workspace, workspace_bytes, stream);
+}
+
 extern "C" int32_t nect_ray_order(const NectGeometry *geometry, const int64_t *ray_index, int64_t n_ray_index,
                                   int32_t num_rays, int32_t starting_ray_index, int32_t *order, void *workspace,
                                   int64_t workspace_bytes, void *stream) {
     clear_error();
     if (check_geometry(geometry)) return 1;
+    return order_rays(patch_key(*geometry), ray_index, n_ray_index, num_rays, starting_ray_index, order, workspace,
+                      workspace_bytes, stream);
+}
+
+static int32_t order_rays(const PatchKey &pk, const int64_t *ray_index, int64_t n_ray_index, int32_t num_rays,
+                          int32_t starting_ray_index, int32_t *order, void *workspace, int64_t workspace_bytes,
+                          void *stream) {
     NECT_REQUIRE(num_rays >= 0 && starting_ray_index >= 0 && n_ray_index >= 0, "negative size or start");
     if (num_rays == 0) return 0;
     NECT_REQUIRE(ray_index && order && workspace, "NULL pointer");
     NECT_REQUIRE(((uintptr_t)workspace & 7) == 0, "workspace must be 8-byte aligned");
-    const PatchKey pk = patch_key(*geometry);
     const int n = pk.n_cells + 1;
     NECT_REQUIRE(workspace_bytes >= 20 * (int64_t)n, "workspace smaller than nect_ray_order_workspace()");
     hipStream_t st = as_stream(stream);
