@@ -3,7 +3,7 @@
 #include <mutex>
 #include <string>
 
-#include "mlp_bwd_twin.hpp"
+#include "mlp_bwd_shared.hpp"
 
 namespace nect {
 
@@ -181,7 +181,7 @@ extern "C" int32_t nect_mlp_forward(const NectMlpDesc *desc, int32_t dtype, cons
 
 // Persistent workgroups: as many as fit on the device at once (two per CU when the LDS image allows).
 static unsigned backward_blocks(const NectMlpDesc *d, int32_t dtype, int64_t n) {
-    if (twin_suits(*d, dtype)) {
+    if (twin_suits(*d, dtype) || shared_suits(*d, dtype)) {
         const int64_t groups = ((n + kTile - 1) / kTile + kTwinWaves - 1) / kTwinWaves;
         return (unsigned)std::min<int64_t>(groups, (int64_t)device_cus() * twin_per_simd(elem_bytes(dtype), *d));
     }
@@ -233,12 +233,14 @@ static int32_t mlp_backward_impl(const NectMlpDesc *desc, int32_t dtype, const v
     const int H = desc->n_hidden_layers;
     const int NQ0 = a.L.PT / 32;
     NECT_REQUIRE(dtype != NECT_F32 || H <= 3, "float32 backward supports at most 3 hidden layers (LDS image)");
-    NECT_REQUIRE(twin_suits(*desc, dtype) || bytes <= kLdsBytes, "network too large for the LDS image of the backward pass");
+    NECT_REQUIRE(bytes <= kLdsBytes, "network too large for the LDS image of the backward pass");
     int32_t rc = 1;
     if (twin_suits(*desc, dtype))
         rc = dtype == NECT_F32   ? launch_mlp_backward_twin_f32(a, blocks, st)
              : dtype == NECT_F16 ? launch_mlp_backward_twin_f16(a, blocks, st)
                                  : launch_mlp_backward_twin_bf16(a, blocks, st);
+    else if (shared_suits(*desc, dtype))
+        rc = dtype == NECT_F16 ? launch_mlp_backward_shared_f16(a, blocks, st) : launch_mlp_backward_shared_bf16(a, blocks, st);
     else if (dtype == NECT_F32) rc = launch_mlp_backward_f32(a, H, NQ0, act_is_pwl(desc->activation), blocks, waves, bytes, st);
     else if (dtype == NECT_F16) rc = launch_mlp_backward_f16(a, H, NQ0, act_is_pwl(desc->activation), blocks, waves, bytes, st);
     else rc = launch_mlp_backward_bf16(a, H, NQ0, act_is_pwl(desc->activation), blocks, waves, bytes, st);

@@ -1,0 +1,13 @@
+// k_mlp_backward_shared instantiations: bf16_t weights, ReLU.
+#include "mlp_bwd_shared.hpp"
+
+namespace nect {
+
+int32_t launch_mlp_backward_shared_bf16_pwl(const MlpArgs &a, unsigned workgroups, hipStream_t st);
+
+int32_t launch_mlp_backward_shared_bf16(const MlpArgs &a, unsigned workgroups, hipStream_t st) {
+    if (a.d.activation != NECT_ACT_RELU) return launch_mlp_backward_shared_bf16_pwl(a, workgroups, st);
+    return launch_mlp_backward_shared<bf16_t, true, 1, 7>(a, workgroups, st);
+}
+
+}  // namespace nect

@@ -22,7 +22,7 @@
 // 0.18, 0.34, 0.44, 0.79); 64 inputs 0.67 -> 0.24, 0.86 -> 0.36, 1.21 -> 0.60,
 // 1.33 -> 1.18; FP32, 32 inputs, 1 to 3 layers 1.56 -> 0.39, 2.44 -> 1.02,
 // 3.38 -> 1.87.  (With five layers the accumulators exceed the register file; four
-// spill some already.)
+// spill some already.  Beyond: k_mlp_backward_shared.)
 #pragma once
 
 #include "mlp_bwd.hpp"
@@ -172,8 +172,8 @@ __device__ __forceinline__ void twin_mask16(const f32x16 &d, const typename Chun
     }
 }
 
-// LDS image of a workgroup (byte offsets): the weights, rows padded by 16 bytes and W0 to 32 NQ0 inputs; per wave its
-// inputs turned (32 NQ0 rows of 32 samples) and dL/dz of the output (float32, and rounded to T); and the row-layout
+// LDS image of a workgroup (byte offsets): the weights, rows padded by 16 bytes and W0 to whole blocks of 32 inputs; per
+// wave its inputs turned (PT rows of 32 samples) and dL/dz of the output (float32, and rounded to T); and the row-layout
 // column of each input.  The parameter gradient is summed over the waves in place of what precedes the columns.
 template <typename T, int H, int NQ0>
 struct TwinLds {
@@ -209,13 +209,15 @@ inline int twin_per_simd(int elem_bytes, const NectMlpDesc &d) {
     return twin_per_simd(elem_bytes, d.n_hidden_layers, (d.n_input_padded + 31) / 32);
 }
 
-template <typename T, int H, int NQ0, bool RELU>
-__global__ __launch_bounds__(64 * kTwinWaves, twin_per_simd((int)sizeof(T), H, NQ0)) void k_mlp_backward_twin(MlpArgs a) {
+// NP: the padded inputs in sixteens.
+template <typename T, int H, int NP, bool RELU>
+__global__ __launch_bounds__(64 * kTwinWaves, twin_per_simd((int)sizeof(T), H, (NP + 1) / 2)) void k_mlp_backward_twin(MlpArgs a) {
     using C = Chunk<T>;
     using chunk = typename C::type;
+    constexpr int NQ0 = (NP + 1) / 2, P = 16 * NP;
     using L = TwinLds<T, H, NQ0>;
     constexpr int V = C::V, N = 16 / V;        // chunks per 16 values
-    constexpr int half = 16 * NQ0;             // inputs of a lane half: half h takes columns half * h ..
+    constexpr int half = 8 * NP;               // inputs of a lane half: half h takes columns half * h ..
     constexpr int NT = half / V;
     constexpr int PT = L::PT, SP = L::SP, SW = L::SW, ST = L::ST;
     extern __shared__ __align__(16) char smem[];
@@ -223,7 +225,6 @@ __global__ __launch_bounds__(64 * kTwinWaves, twin_per_simd((int)sizeof(T), H, N
     T *w0t = reinterpret_cast<T *>(smem + L::w0t), *wht = reinterpret_cast<T *>(smem + L::wht);
     float *wo = reinterpret_cast<float *>(smem + L::wo);
     int *cmap = reinterpret_cast<int *>(smem + L::cmap);
-    const int P = a.d.n_input_padded;
     {
         const T *W = static_cast<const T *>(a.w);
         for (int e = threadIdx.x; e < kWidth * PT; e += blockDim.x) {
@@ -251,6 +252,8 @@ __global__ __launch_bounds__(64 * kTwinWaves, twin_per_simd((int)sizeof(T), H, N
     char *mine = smem + L::scratch + wave * L::per_wave;
     T *XT = reinterpret_cast<T *>(mine);                    // [input column][sample]
     float *go_row = reinterpret_cast<float *>(mine + L::go);
+    for (int i = P; i < PT; ++i)
+        if (lane < ST) XT[i * ST + lane] = zero_of<T>();
     __syncthreads();
 
     const float loss_scale = a.loss_scale_dev ? a.loss_scale_dev[0] : a.loss_scale;
@@ -258,7 +261,7 @@ __global__ __launch_bounds__(64 * kTwinWaves, twin_per_simd((int)sizeof(T), H, N
     const float slope = act_pwl_slope(a.d.activation);
     // a lane's inputs as pieces of 8 bytes: whole rows, or planes of half a chunk or of whole chunks
     const int vpp = a.x_vpp;
-    const bool pieces = P == PT && (vpp ? vpp == V / 2 || vpp % V == 0 : a.x_vec && a.d.n_input == P);
+    const bool pieces = (vpp ? vpp == V / 2 || vpp % V == 0 : a.x_vec && a.d.n_input == P);
     const int64_t second = vpp == V / 2 ? a.x_plane : V / 2;
     int64_t xoff[NT];
 #pragma unroll
@@ -531,21 +534,26 @@ int32_t launch_mlp_backward_twin_f16(const MlpArgs &a, unsigned workgroups, hipS
 int32_t launch_mlp_backward_twin_bf16(const MlpArgs &a, unsigned workgroups, hipStream_t st);
 int32_t launch_mlp_backward_twin_f32(const MlpArgs &a, unsigned workgroups, hipStream_t st);
 
-template <typename T, int H, int NQ0>
+template <typename T, int H, int NP>
 int32_t launch_mlp_backward_twin_as(const MlpArgs &a, unsigned workgroups, hipStream_t st) {
-    constexpr size_t bytes = TwinLds<T, H, NQ0>::total;
+    constexpr size_t bytes = TwinLds<T, H, (NP + 1) / 2>::total;
     static_assert(bytes <= kLdsLimit, "LDS image too large");
     return a.d.activation == NECT_ACT_RELU
-               ? launch_with_lds(k_mlp_backward_twin<T, H, NQ0, true>, workgroups, 64 * kTwinWaves, bytes, st, a, "k_mlp_backward_twin")
-               : launch_with_lds(k_mlp_backward_twin<T, H, NQ0, false>, workgroups, 64 * kTwinWaves, bytes, st, a, "k_mlp_backward_twin");
+               ? launch_with_lds(k_mlp_backward_twin<T, H, NP, true>, workgroups, 64 * kTwinWaves, bytes, st, a, "k_mlp_backward_twin")
+               : launch_with_lds(k_mlp_backward_twin<T, H, NP, false>, workgroups, 64 * kTwinWaves, bytes, st, a, "k_mlp_backward_twin");
 }
 
 template <typename T, int H0, int H1>
 int32_t launch_mlp_backward_twin(const MlpArgs &a, unsigned workgroups, hipStream_t st) {
     if constexpr (H0 <= H1) {
-        if (a.d.n_hidden_layers == H0)
-            return a.d.n_input_padded <= 32 ? launch_mlp_backward_twin_as<T, H0, 1>(a, workgroups, st)
-                                            : launch_mlp_backward_twin_as<T, H0, 2>(a, workgroups, st);
+        if (a.d.n_hidden_layers == H0) {
+            switch (a.d.n_input_padded / 16) {
+                case 1: return launch_mlp_backward_twin_as<T, H0, 1>(a, workgroups, st);
+                case 2: return launch_mlp_backward_twin_as<T, H0, 2>(a, workgroups, st);
+                case 3: return launch_mlp_backward_twin_as<T, H0, 3>(a, workgroups, st);
+                default: return launch_mlp_backward_twin_as<T, H0, 4>(a, workgroups, st);
+            }
+        }
         return launch_mlp_backward_twin<T, H0 + 1, H1>(a, workgroups, st);
     } else {
         set_error("k_mlp_backward_twin: no instantiation for this depth");
