@@ -183,7 +183,8 @@ extern "C" int32_t nect_mlp_forward(const NectMlpDesc *desc, int32_t dtype, cons
 static unsigned backward_blocks(const NectMlpDesc *d, int32_t dtype, int64_t n) {
     if (twin_suits(*d, dtype) || shared_suits(*d, dtype)) {
         const int64_t groups = ((n + kTile - 1) / kTile + kTwinWaves - 1) / kTwinWaves;
-        return (unsigned)std::min<int64_t>(groups, (int64_t)device_cus() * twin_per_simd(elem_bytes(dtype), *d));
+        const int per_cu = twin_suits(*d, dtype) ? twin_per_simd(elem_bytes(dtype), *d) : 1;
+        return (unsigned)std::min<int64_t>(groups, (int64_t)device_cus() * per_cu);
     }
     const int waves = waves_per_block(dtype, true);
     const int64_t groups = ((n + kTile - 1) / kTile + waves - 1) / waves;

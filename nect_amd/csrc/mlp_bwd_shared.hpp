@@ -240,7 +240,7 @@ __global__ __launch_bounds__(64 * kTwinWaves, 1) void k_mlp_backward_shared(MlpA
                     float v[V], z[V];
 #pragma unroll
                     for (int m = 0; m < V; ++m) {
-                        v[m] = wo[32 * p + acc_row(V * c + m, h)] * gs;
+                        v[m] = as_float32(wo[32 * p + acc_row(V * c + m, h)] * gs);
                         z[m] = z1[p][V * c + m];
                     }
                     g1[p][c] = twin_mask<T, RELU>(v, z, slope);
@@ -260,7 +260,7 @@ __global__ __launch_bounds__(64 * kTwinWaves, 1) void k_mlp_backward_shared(MlpA
                     float v[V], z[V];
 #pragma unroll
                     for (int m = 0; m < V; ++m) {
-                        v[m] = w * go2[m];
+                        v[m] = as_float32(w * go2[m]);
                         z[m] = twin_act<RELU>(z2[p][V * c + m], slope);
                     }
                     // (the operands of a weight gradient are rounded to T, here as in the other layers)

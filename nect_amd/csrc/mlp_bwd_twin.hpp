@@ -18,8 +18,8 @@
 // products of the one or two waves per SIMD that its accumulators leave room for.
 //
 // 2^21 samples, k_mlp_backward -> this kernel, ms: 32 inputs, FP16, ReLU, 1, 2, 3 and
-// 4 hidden layers 0.36 -> 0.14, 0.40 -> 0.28, 0.81 -> 0.38, 0.94 -> 0.68 (LeakyReLU
-// 0.18, 0.34, 0.44, 0.79); 64 inputs 0.67 -> 0.24, 0.86 -> 0.36, 1.21 -> 0.60,
+// 4 hidden layers 0.36 -> 0.14, 0.40 -> 0.31, 0.81 -> 0.39, 0.94 -> 0.68 (LeakyReLU
+// 0.18, 0.35, 0.44, 0.79); 64 inputs 0.67 -> 0.24, 0.86 -> 0.39, 1.21 -> 0.53,
 // 1.33 -> 1.18; FP32, 32 inputs, 1 to 3 layers 1.56 -> 0.39, 2.44 -> 1.02,
 // 3.38 -> 1.87.  (With five layers the accumulators exceed the register file; four
 // spill some already.  Beyond: k_mlp_backward_shared.)
@@ -107,6 +107,12 @@ __device__ __forceinline__ void twin_act16(const f32x16 &z, float slope, typenam
     }
 }
 
+// A product as rounded to float32: its conversion to float16 is not folded into it (v_fma_mixlo_f16 rounds once).
+__device__ __forceinline__ float as_float32(float v) {
+    __asm__("" : "+v"(v));
+    return v;
+}
+
 // v where the signed 16-bit halves of `a` are positive, else slope * v (RELU: 0), as a chunk of 16-bit values.  Whole
 // halves of packed results are chosen: 0 - a, saturated, is negative where a > 0, and v_perm_b32 spreads its sign over
 // the half -- no comparison per value, and half the registers of one.
@@ -118,7 +124,7 @@ __device__ __forceinline__ typename Chunk<T>::type twin_choose(const float (&v)[
     if constexpr (!RELU) {
         float b[8];
 #pragma unroll
-        for (int m = 0; m < 8; ++m) b[m] = v[m] * slope;
+        for (int m = 0; m < 8; ++m) b[m] = as_float32(v[m] * slope);
         below = __builtin_bit_cast(u32x4, Chunk<T>::pack(b));
     }
     u32x4 r;
@@ -200,18 +206,19 @@ inline bool twin_suits(const NectMlpDesc &d, int32_t dtype) {
     return d.n_output == 1 && act_is_pwl(d.activation) && NQ0 <= 2 && H <= (dtype == NECT_F32 ? 3 : 4);
 }
 
-// Waves per SIMD (workgroups per CU): the accumulators of two hidden layers and 32 inputs leave room for two (0.31 ms; with
-// one 0.33); with 64 inputs two would spill (0.63 ms; one 0.38).
-__host__ __device__ constexpr int twin_per_simd(int elem_bytes, int H, int NQ0) {
-    return elem_bytes == 2 && twin_blocks(H, NQ0) <= 6 ? 2 : 1;
+// Waves per SIMD (workgroups per CU): the accumulators of two hidden layers and 32 inputs leave room for two with a ReLU
+// (0.31 ms; with one 0.33), of one layer with the others, whose slope costs registers (two layers 0.42; one wave 0.34);
+// with 64 inputs and two layers two waves would spill (0.63 ms; one 0.38).
+__host__ __device__ constexpr int twin_per_simd(int elem_bytes, int H, int NQ0, bool relu) {
+    return elem_bytes == 2 && twin_blocks(H, NQ0) <= (relu ? 6 : 4) ? 2 : 1;
 }
 inline int twin_per_simd(int elem_bytes, const NectMlpDesc &d) {
-    return twin_per_simd(elem_bytes, d.n_hidden_layers, (d.n_input_padded + 31) / 32);
+    return twin_per_simd(elem_bytes, d.n_hidden_layers, (d.n_input_padded + 31) / 32, d.activation == NECT_ACT_RELU);
 }
 
 // NP: the padded inputs in sixteens.
 template <typename T, int H, int NP, bool RELU>
-__global__ __launch_bounds__(64 * kTwinWaves, twin_per_simd((int)sizeof(T), H, (NP + 1) / 2)) void k_mlp_backward_twin(MlpArgs a) {
+__global__ __launch_bounds__(64 * kTwinWaves, twin_per_simd((int)sizeof(T), H, (NP + 1) / 2, RELU)) void k_mlp_backward_twin(MlpArgs a) {
     using C = Chunk<T>;
     using chunk = typename C::type;
     constexpr int NQ0 = (NP + 1) / 2, P = 16 * NP;
@@ -380,7 +387,7 @@ __global__ __launch_bounds__(64 * kTwinWaves, twin_per_simd((int)sizeof(T), H, (
                     float v[V], z[V];
 #pragma unroll
                     for (int m = 0; m < V; ++m) {
-                        v[m] = wo[32 * p + acc_row(V * c + m, h)] * gs;
+                        v[m] = as_float32(wo[32 * p + acc_row(V * c + m, h)] * gs);
                         z[m] = z1[p][V * c + m];
                     }
                     g1[p][c] = twin_mask<T, RELU>(v, z, slope);
@@ -400,7 +407,7 @@ __global__ __launch_bounds__(64 * kTwinWaves, twin_per_simd((int)sizeof(T), H, (
                     float v[V], z[V];
 #pragma unroll
                     for (int m = 0; m < V; ++m) {
-                        v[m] = w * go2[m];
+                        v[m] = as_float32(w * go2[m]);
                         z[m] = twin_act<RELU>(z2[p][V * c + m], slope);
                     }
                     // (the operands of a weight gradient are rounded to T, here as in the other layers)

@@ -158,3 +158,25 @@ def test_not_finite(device, act, value):
     keep = torch.arange(500, device=device) != 77
     assert torch.equal(res[0][1][keep], res[1][1][keep])
     assert bool(torch.isfinite(res[0][0]).all()) and not bool(torch.isfinite(res[1][0]).all())
+
+
+@pytest.mark.parametrize("act", ["ReLU", "LeakyReLU"])
+def test_float16_rounding(device, act):
+    """dL/dz is the product rounded to float32 and then to float16: with W0 a permutation, dL/dx is dL/dz itself, bit for bit."""
+    from nect_amd.mlp import MlpDesc, backward
+
+    d = MlpDesc(64, 1, 64, 1, act, "None")
+    g = torch.Generator().manual_seed(4)
+    n = 100_000
+    wo = torch.randn(64, generator=g).half()
+    w = torch.zeros(d.n_params, dtype=torch.float16)
+    w[:4096] = torch.eye(64).half().flatten()
+    w[4096:4160] = wo
+    x = (torch.randn(n, 64, generator=g)).half()
+    dy = torch.randn(n, 1, generator=g)
+    dw, dx = torch.zeros(d.n_params, device=device), torch.zeros((n, 64), device=device)
+    backward(d, w.to(device), x.to(device), dy.to(device), dw, dx, loss_scale=1.0, grad_scale=1.0)
+    torch.cuda.synchronize()
+    p = dy * wo.float()
+    below = p * 0.01 if act == "LeakyReLU" else torch.zeros_like(p)
+    assert torch.equal(dx.cpu(), torch.where(x > 0, p, below).half().float())
