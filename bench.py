@@ -133,10 +133,8 @@ def parse():
     ap.add_argument("--static-preset-only", action="store_true",
                     help="only the training step of the reference's default static model (hash_grid preset)")
     ap.add_argument("--scatter-split", action="store_true",
-                    help="with --quadcubes-only: the scatter's LDS-aggregated and direct levels as two launches each "
-                         "(to time the phases apart)")
-    ap.add_argument("--atomic-file", default=os.path.join(ROOT, "profiles", "atomic_rate.json"),
-                    help="the atomic request rate measured by --atomic-calibration (optional)")
+                    help="with --quadcubes-only: the ray-group scatter (instead of the binned one), its LDS-aggregated "
+                         "and direct levels as two launches each (to time the phases apart)")
     ap.add_argument("--query-only", action="store_true",
                     help="only the 512^3 export volume of the serving model (e.g. under a profiler)")
     ap.add_argument("--summarize-pmc", nargs="+", metavar="CSV",
@@ -413,20 +411,6 @@ def main():
                 "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
                 "algorithmic_bytes_per_launch": per_sample_bytes[dominant] * n_samples,
                 "samples_per_launch": n_samples}
-    if dominant == "grid_backward" and measured.get("grid_backward_atomic_requests"):
-        # the bound this kernel meets: atomic requests (one per 64-byte block per wave instruction), counted by
-        # TCC_EA0_ATOMIC_sum on the same workload, against the request rate --atomic-calibration measured
-        req = measured["grid_backward_atomic_requests"]
-        rate = req / (kernels[dominant] / 1e3) / 1e9
-        try:
-            with open(args.atomic_file) as f:
-                peak = float(json.load(f)["requests_per_s_G"])
-        except (OSError, ValueError, KeyError):
-            peak = None
-        roofline["atomic_requests"] = {"per_launch": req, "achieved": round(rate, 2), "peak": peak,
-                                       "unit": "G requests/s",
-                                       "frac": round(rate / peak, 3) if peak else None}
-
     # every kernel of the step against its own roofline (algorithmic work / mean launch time)
     H = mlp.n_hidden_layers
     mlp_fwd_flop = 2 * (mlp.n_input * mlp.width + (H - 1) * mlp.width * mlp.width + mlp.width * mlp.n_output)
@@ -780,8 +764,8 @@ def quadcubes_step(dev, steps: int = 5, S: int = 256, points_per_batch: int = 5_
     <= 256 -- with the L1 loss of cfg/default.yaml, on the 4D workload's geometry and brine-front projections
     (Views4D).  Trained through ModuleTrainStep: patch-ordered
     batch, nested grids encoded in one launch, the layers as nect_gemm_act products with their activations and
-    k_wgrad weight gradients, ray-group scatter per grid, dense Adam.  split: each grid's scatter as two launches
-    (LDS-aggregated levels, then the direct levels), to time the phases apart."""
+    k_wgrad weight gradients, binned scatter per grid, dense Adam.  split: the ray-group scatter instead, each
+    grid's as two launches (LDS-aggregated levels, then the direct levels), to time the phases apart."""
     from nect_amd.module_step import ModuleTrainStep
     from nect_amd.networks import QuadCubes
     from nect_amd.sampling.geometry import Geometry
@@ -799,7 +783,8 @@ def quadcubes_step(dev, steps: int = 5, S: int = 256, points_per_batch: int = 5_
     model = QuadCubes(enc, net, include_identity=True, dtype=torch.float16).to(dev)
     B = (points_per_batch // 2) // S
     st = ModuleTrainStep(model, torch.float16, B, S, loss="L1", dynamic=True)
-    st.scatter_split = split
+    if split:
+        st.scatter, st.scatter_split = "groups", True
     gen = torch.Generator(device=dev).manual_seed(21)
     print("[bench] QuadCubes preset", file=sys.stderr, flush=True)
     views = Views4D(dev, geo, n_views)

@@ -151,7 +151,7 @@ __global__ __launch_bounds__(256) void k_grid_encode_pair(NectGridDesc g, const 
 // by the cache lines an instruction touches, then touch a fraction of those that
 // 32 samples along one ray do.  Encoder of one step, k_grid_encode_pair in patch
 // order -> this kernel in column order: 262144 x 256 samples, 16 levels, FP16
-// 3.04 -> 1.62 ms; 4-D BF16 7.73 -> 5.76; 20 levels of 4 features 1.06 -> 0.65;
+// 3.04 -> 1.62 ms; 4-D BF16 7.73 -> 5.76; 19 levels of 4 features 1.06 -> 0.65;
 // FP32 0.83 -> 0.50; below about 8192 rays of 128 samples the other way round
 // (1024 x 64: 0.021 -> 0.050 ms, too few waves in flight).
 // PLANAR: the level-grouped schedule and planes of k_grid_encode_pair; else one
