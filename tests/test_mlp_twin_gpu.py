@@ -180,3 +180,28 @@ def test_float16_rounding(device, act):
     p = dy * wo.float()
     below = p * 0.01 if act == "LeakyReLU" else torch.zeros_like(p)
     assert torch.equal(dx.cpu(), torch.where(x > 0, p, below).half().float())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("hidden,act,n_in", [(6, "LeakyReLU", 76), (5, "ReLU", 32), (2, "ReLU", 128), (3, "LeakyReLU", 32)])
+@pytest.mark.parametrize("tiles", [1, 6, 7, 8, 1029, 1030, 1031])
+def test_rows_past_the_count(device, dtype, hidden, act, n_in, tiles):
+    """Rows of the tiles past the count on the device hold whatever their memory held: with NaN and infinities there, the
+    weight gradient is bit for bit that of zeros there, also where a workgroup's waves have 1, 2 or 3 live tiles."""
+    from nect_amd.mlp import MlpDesc, backward
+
+    print(f"[twin] past the count {dtype} H={hidden} {act} in={n_in} tiles={tiles}", flush=True)
+    n, rows = 32 * (tiles + 5), 32 * tiles
+    d = MlpDesc(n_in, 1, 64, hidden, act, "None")
+    w, x, dy = (v.to(device) for v in case(d, dtype, n, tiles))
+    count = torch.tensor([tiles], dtype=torch.int32, device=device)
+    res = []
+    for value in (0.0, float("nan"), float("inf"), -float("inf")):
+        x[rows:], dy[rows:] = value, value
+        dw = torch.zeros(d.n_params, device=device)
+        backward(d, w, x, dy, dw, None, n_tiles_dev=count, loss_scale=256.0 * n, grad_scale=1.0)
+        torch.cuda.synchronize()
+        res.append(dw)
+    assert bool(torch.isfinite(res[0]).all()) and bool(res[0].any())
+    for dw in res[1:]:
+        assert torch.equal(dw, res[0])

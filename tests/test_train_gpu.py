@@ -486,3 +486,39 @@ def test_fp16_step_skips_non_finite_gradient_and_backs_off(device):
     assert st2["scale"] == st1["scale"] * 2
     assert not torch.equal(fs.params, snap[0])
     assert torch.isfinite(fs.params).all() and torch.isfinite(fs.shadow.float()).all()
+
+
+def test_unwritten_feature_rows_do_not_reach_the_gradient(device):
+    """The step's feature rows past the batch's tiles are never written: whatever they hold, no step of the six-layer
+    76-input model is skipped and its gradient is finite (batches whose tiles are no multiple of 4 among them)."""
+    from nect_amd.fused import FusedTrainStep, init_params
+    from nect_amd.grid import GridDesc
+    from nect_amd.mlp import MlpDesc
+
+    print("[train] unwritten feature rows", flush=True)
+    g = cfg1_geometry()
+    geo = product_struct(g.c_struct_fields())
+    S = 64
+    step = g.max_distance_traveled / S
+    grid = GridDesc(3, 19, 4, 12, 8, 1.26)
+    mlp = MlpDesc(76, 1, 64, 6, "LeakyReLU", "ReLU")
+    params = init_params(grid, mlp, seed=5, device=device)
+    gen = torch.Generator().manual_seed(6)
+    params[mlp.n_params:] = ((torch.rand(grid.n_params, generator=gen) * 2 - 1) * 0.5).to(device)
+    fs = FusedTrainStep(grid, mlp, params, torch.float16, max_rays=512, max_points_per_ray=S, loss="L1")
+    idx, jit, off = (torch.from_numpy(a).to(device) for a in seeded_batch(64 * 64, 512, seed=3))
+    tgt = torch.full((512,), 0.3, device=device)
+    left = set()
+    for k, B in enumerate([101, 300, 307, 311, 313, 317, 331, 512]):
+        fs.features.fill_(float("nan") if k % 2 == 0 else float("inf"))
+        fs.step(geo, 0.5, idx, 0, B, S, step, True, jit, off, tgt[:B], g.max_distance_traveled, lr=0.0,
+                optimizer_step=False)
+        torch.cuda.synchronize()
+        tiles = int(fs.n_tiles.item())
+        assert tiles < 2 * B
+        left.add(tiles % 4)
+        assert bool(torch.isfinite(fs.grad).all()), (B, tiles)
+        assert bool(fs.grad[:mlp.n_params].any())
+        fs.adam(1e-3)
+    assert len(left - {0}) >= 2, left
+    assert fs.amp_status()["skipped"] == 0 and fs.amp_status()["step"] == 8
