@@ -564,6 +564,9 @@ enum NectRescale {
                                          (create_volume of a half-precision model) */
 };
 
+/* Added to NectQueryJob.brick: the bricks stacked along z. */
+#define NECT_BRICK_STACKED 0x1000
+
 /*
  * One chunk of an export query (nect/static_export.py:106-141,
  * nect/dynamic_export.py:519-537, nect/trainers/base_trainer.py:402-450):
@@ -573,7 +576,12 @@ enum NectRescale {
  * (each 0..4) names bricks of 2^bz x 2^by x 2^bx voxels that tile the grid
  * padded up to whole bricks: position v is voxel v mod 2^(bz+by+bx) (row order
  * inside the brick) of brick v >> (bz+by+bx) (row order over the bricks);
- * positions in the padding are skipped.  Neighbouring voxels are then
+ * positions in the padding are skipped.  With NECT_BRICK_STACKED added to the
+ * code the bricks are taken in layers of min(32 >> bz, bricks along z) of them
+ * stacked along z (the last layer may be thinner), a layer's stacks in row order
+ * over (y, x), a stack's voxels with z fastest, then x, then y: twice as fast
+ * (consecutive positions then lie along z, the table's contiguous coordinate),
+ * and the order to cut a grid into chunks by.  Neighbouring voxels are then
  * evaluated together, so their shared hash-table entries are read once from
  * HBM; the traversal length is the padded voxel count.  Every voxel is written
  * at out[(iz*n[1] + iy)*n[2] + ix] (out is the whole grid's output, in the
@@ -597,7 +605,7 @@ typedef struct NectQueryJob {
     float lo;
     int32_t mu_dtype;       /* NECT_F32 or NECT_F16 */
     int32_t rescale;        /* NectRescale */
-    int32_t brick;          /* traversal: 0 = row order, else (bz << 8) | (by << 4) | bx */
+    int32_t brick;          /* traversal: 0 = row order, else (bz << 8) | (by << 4) | bx [| NECT_BRICK_STACKED] */
     const float *axis[3];   /* optional explicit coordinates (z, y, x) */
     int64_t v0;
     int64_t count;

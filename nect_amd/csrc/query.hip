@@ -35,9 +35,11 @@ __device__ __forceinline__ float rescale_value(const NectQueryJob &J, float mu) 
 
 // Voxel (iz, iy, ix) at traversal position v of a job's grid; false for positions
 // in the padding or past the grid.  Row order, or (J.brick) the grid padded to
-// whole bricks of 2^lz x 2^ly x 2^lx voxels, taken in layers of bricks stacked up
-// to 32 voxels along z; a layer column by column, a column (one stack of bricks)
-// with z fastest, then x, then y.
+// whole bricks of 2^lz x 2^ly x 2^lx voxels: in row order, their voxels in row
+// order, or (NECT_BRICK_STACKED, and a job that takes the whole traversal, where
+// the order is nobody's business) in layers of bricks stacked up to 32 voxels
+// along z; a layer column by column, a column (one stack of bricks) with z
+// fastest, then x, then y.
 // z is the grid's first coordinate, whose neighbouring cells are neighbouring
 // table entries on dense and hashed levels alike (its stride or prime is 1), so
 // a wave whose 32 voxels lie along z gathers from a fraction of the cache lines,
@@ -64,6 +66,15 @@ __device__ __forceinline__ bool query_voxel(const NectQueryJob &J, int64_t v, in
     const uint32_t nby = ((uint32_t)J.n[1] + (1u << ly) - 1u) >> ly;
     const uint32_t nbz = ((uint32_t)J.n[0] + (1u << lz) - 1u) >> lz;
     const uint32_t plane = nby * nbx;
+    if (!(J.brick & NECT_BRICK_STACKED) && (J.v0 != 0 || J.count < ((int64_t)(nbz * plane) << ib))) {
+        const uint32_t bz = b / plane;
+        const uint32_t r = b - bz * plane;
+        const uint32_t by = r / nbx;
+        iz = (int32_t)((bz << lz) + (in >> (ly + lx)));
+        iy = (int32_t)((by << ly) + ((in >> lx) & ((1u << ly) - 1u)));
+        ix = (int32_t)(((r - by * nbx) << lx) + (in & ((1u << lx) - 1u)));
+        return iz < J.n[0] && iy < J.n[1] && ix < J.n[2];
+    }
     const uint32_t stack = min(32u >> lz, nbz);      // bricks per column of a layer (fewer in the last one)
     const uint32_t layer = b / (stack * plane);
     const uint32_t z0 = layer * stack;

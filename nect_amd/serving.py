@@ -40,6 +40,9 @@ JOB_DTYPE = np.dtype([("n", "<i4", 3), ("a", "<f4", 3), ("b", "<f4", 3), ("t", "
                       ("axis", "<u8", 3), ("v0", "<i8"), ("count", "<i8"), ("out", "<u8")])
 assert JOB_DTYPE.itemsize == 112
 
+# NECT_BRICK_STACKED: the bricks of a traversal stacked along z
+BRICK_STACKED = 0x1000
+
 # NectRescale: how the network output becomes a voxel value, ((mu / l_max) * span) + lo
 RESCALE_DIVIDE, RESCALE_RECIPROCAL, RESCALE_RECIPROCAL_F16 = 0, 1, 2
 
@@ -211,7 +214,7 @@ class QueryServer:
             jobs[k]["lo"] = r.lo
             jobs[k]["mu_dtype"] = _lib.F16 if r.mu_half else _lib.F32
             jobs[k]["rescale"] = r.rescale
-            jobs[k]["brick"] = r.brick
+            jobs[k]["brick"] = r.brick | BRICK_STACKED if r.brick else 0
             if r.axes is not None:
                 for d in range(3):
                     ax = r.axes[d]

@@ -245,3 +245,46 @@ def test_create_volume_matches_oracle(device):
     ref = oq.rescale(mu, geo.max_distance_traveled, span, float(proj.min()), "reciprocal_f16", "float16")
     assert vol.shape == (12, 10, 8)
     assert np.array_equal(vol.ravel(), ref)
+
+
+@pytest.mark.parametrize("n", [(70, 9, 11), (37, 6, 5), (33, 33, 1), (7, 18, 33)])
+@pytest.mark.parametrize("code", [0x222, 0x000, 0x410, 0x124, 0x044, 0x301])
+@pytest.mark.parametrize("stacked", [False, True])
+def test_chunks_take_the_voxels_of_their_positions(device, n, code, stacked):
+    """A job of the positions [v0, v0 + count) writes the voxels that the header says lie there, in row order of the
+    bricks and stacked along z, and no others, with the values that row order gives; grids that are no multiple of a
+    brick, and of 32 along z."""
+    from nect_amd import _lib
+    from nect_amd.serving import BRICK_STACKED, JOB_DTYPE
+    from tests.test_serving_cpu import _stacked_voxels, _voxels
+
+    print(f"[query] chunks {n} code={code:#x} stacked={stacked}", flush=True)
+    grid, mlp, w, tab, _, _ = model(device, torch.float16)
+    lg = ((code >> 8) & 15, (code >> 4) & 15, code & 15)
+    length = int(np.prod([-(-k // (1 << l)) for k, l in zip(n, lg)])) << sum(lg)
+    vox = int(np.prod(n))
+
+    def run(brick, v0, count):
+        out = torch.full((vox,), -7.0, device=device)
+        job = np.zeros(1, JOB_DTYPE)
+        job["n"], job["b"], job["l_max"], job["span"] = n, 1.0, 1.0, 1.0
+        job["brick"], job["v0"], job["count"], job["out"] = brick, v0, count, out.data_ptr()
+        jobs = torch.from_numpy(job.view(np.uint8)).to(device)
+        pref = torch.tensor([0, (count + 31) // 32], dtype=torch.int64, device=device)
+        _lib.call("nect_query", grid.struct_ref(), mlp.struct_ref(), _lib.F16, w.data_ptr(), tab.data_ptr(),
+                  jobs.data_ptr(), pref.data_ptr(), 1, (count + 31) // 32, _lib.F32, _lib.stream_of(device))
+        torch.cuda.synchronize()
+        return out.cpu().numpy()
+
+    ref = run(0, 0, vox)
+    assert (ref != -7.0).all()
+    use_stacked = stacked and code
+    iz, iy, ix, ok = (_stacked_voxels if use_stacked else _voxels)(n, code, length)
+    flat = (iz * n[1] + iy) * n[2] + ix
+    brick = code | (BRICK_STACKED if use_stacked else 0)
+    for v0, count in [(0, length), (0, length // 3 + 1), (length // 3 + 1, length // 2), (length - 5, 5), (1, 1)]:
+        got = run(brick, v0, count)
+        want = np.full(vox, -7.0, np.float32)
+        at = flat[v0:v0 + count][ok[v0:v0 + count]]
+        want[at] = ref[at]
+        assert np.array_equal(got, want), (v0, count)

@@ -43,3 +43,26 @@ def test_traversal_covers_every_voxel_once():
         # a position past the traversal maps outside the grid
         iz2, iy2, ix2, ok2 = _voxels(n, code, length + 64)
         assert not ok2[length:].any()
+
+
+def _stacked_voxels(n, code, length):
+    """As _voxels for NECT_BRICK_STACKED: layers of bricks stacked up to 32 voxels along z, z fastest in a stack."""
+    lz, ly, lx = (code >> 8) & 15, (code >> 4) & 15, code & 15
+    nbz, nby, nbx = (-(-k // (1 << l)) for k, l in zip(n, (lz, ly, lx)))
+    order = []
+    for z0 in range(0, nbz, 32 >> lz):
+        nz = min(32 >> lz, nbz - z0) << lz
+        y, x, yy, xx, zz = np.meshgrid(np.arange(nby), np.arange(nbx), np.arange(1 << ly), np.arange(1 << lx),
+                                       np.arange(nz), indexing="ij")
+        order.append(np.stack([(z0 << lz) + zz, (y << ly) + yy, (x << lx) + xx], -1).reshape(-1, 3))
+    iz, iy, ix = np.concatenate(order)[:length].T
+    return iz, iy, ix, (iz < n[0]) & (iy < n[1]) & (ix < n[2])
+
+
+def test_stacked_traversal_covers_every_voxel_once():
+    for n in [(7, 33, 40), (1, 512, 9), (5, 1, 3), (65, 66, 67), (37, 5, 6), (4, 4, 4), (2, 3, 17)]:
+        code, length = traversal(n)
+        iz, iy, ix, ok = _stacked_voxels(n, code, length)
+        assert iz.size == length
+        flat = (iz[ok] * n[1] + iy[ok]) * n[2] + ix[ok]
+        assert np.array_equal(np.sort(flat), np.arange(n[0] * n[1] * n[2])), n
