@@ -889,8 +889,16 @@ static int32_t launch_encode_columns(const NectGridDesc &g, int32_t dtype, const
     NECT_REQUIRE((units + 3) / 4 * G < ((int64_t)1 << 31), "too many ray groups");
     const dim3 grid((unsigned)((units + 3) / 4 * G)), block(256);
 #define NECT_ENCC(D, F, T, P)                                                                                       \
-    hipLaunchKernelGGL((k_grid_encode_columns<D, F, T, P>), grid, block, lds, st, g, (const T *)table, rays,         \
-                       tile_offsets, num_rays, n_passes, t, (T *)out, out_stride, G, n_slots, width, ch, vec)
+    do {                                                                                                            \
+        const auto k = k_grid_encode_columns<D, F, T, P>;                                                           \
+        if (lds > 64 * 1024 && hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize,     \
+                                                   (int)lds) != hipSuccess) {                                       \
+            set_error("k_grid_encode_columns: cannot reserve LDS");                                                 \
+            return 1;                                                                                               \
+        }                                                                                                           \
+        hipLaunchKernelGGL(k, grid, block, lds, st, g, (const T *)table, rays, tile_offsets, num_rays, n_passes, t, \
+                           (T *)out, out_stride, G, n_slots, width, ch, vec);                                       \
+    } while (0)
 #define NECT_ENCC_P(D, F, T)                       \
     do {                                           \
         if (planar) NECT_ENCC(D, F, T, true);      \

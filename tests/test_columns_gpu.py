@@ -100,3 +100,9 @@ def test_order(device, rows, cols, unique):
         sel = patch == p
         if len(np.unique(pix[sel])) == sel.sum():
             assert np.all(np.diff(row[sel]) > 0), p
+
+
+@pytest.mark.parametrize("B,S,order", [(33, 32, True), (700, 61, False)])
+def test_encode_widest_float32(device, B, S, order):
+    """32 levels of 4 float32 features: one sample of 512 bytes staged at a time takes more than 64 KiB of LDS."""
+    test_encode_matches(device, (3, 32, 4, 11, 4, 1.15), torch.float32, B, S, order)
