@@ -684,11 +684,12 @@ static int64_t plan_bins(const NectGridDesc &g, bool fold, int64_t slots, BinPla
     const int dims = g.n_dims - (fold ? 1 : 0);
     const int64_t pairs = slots << (dims - 1);
     // small batches (a few rays, a region) crowd into few bins more often, and lists that hold the whole batch cost
-    // them little: within kWholeListBytes in all, no list can overflow
+    // them little: within kWholeListBytes in all, no list can overflow.  (Taken for the grid as it is, folded or not: a
+    // folded batch then never needs more than the same chunks of the unfolded one, which the workspace is sized for.)
     int64_t all = 0;
     for (int l = 0; l < g.n_levels; ++l) {
         const int lb = std::max(0, ceil_log2(g.level_size[l]) - (kBinLog2Floats - (g.n_features == 2 ? 1 : 2)));
-        all += (pairs << lb) * (8 + 4 * g.n_features);
+        all += (slots << (g.n_dims - 1 + lb)) * (8 + 4 * g.n_features);
     }
     const bool whole = all <= kWholeListBytes;
     // a list per XCD once every XCD has many workgroups of the chunk (their shares are even then)
@@ -760,12 +761,13 @@ static int64_t plan_bins(const NectGridDesc &g, bool fold, int64_t slots, BinPla
     return rec;
 }
 
-// Chunks so that counters and records fit in `bytes`; 0 when they cannot.
+// Chunks so that counters and records fit in `bytes`; 0 when they cannot.  The counts tried do not depend on `bytes`, so
+// that the size found for one limit is enough for the launch, whose limit it is.
 static int plan_chunks(const NectGridDesc &g, bool fold, int64_t slots, int64_t bytes, BinPlan &P, int &group_bins,
                        int64_t &chunk_slots, int64_t &need) {
     const int64_t rec_bytes = 8 + 4 * g.n_features;
     const int64_t tiles = (slots + kTile - 1) / kTile;
-    for (int64_t k = 1; k <= tiles && k <= 4096;) {
+    for (int64_t k = 1; k <= tiles && k <= 4096; k += std::max<int64_t>(1, k / 16)) {
         chunk_slots = ((tiles + k - 1) / k) * kTile;
         const int64_t rec = plan_bins(g, fold, chunk_slots, P, group_bins);
         if (rec < 0) return 0;
@@ -774,7 +776,6 @@ static int plan_chunks(const NectGridDesc &g, bool fold, int64_t slots, int64_t 
             P.n_chunks = (int32_t)k;
             return (int)k;
         }
-        k = std::max(k + 1, (int64_t)((double)k * need / bytes * 0.98));
     }
     return 0;
 }
@@ -854,7 +855,7 @@ extern "C" int64_t nect_grid_binned_workspace(const NectGridDesc *desc, int64_t 
     BinPlan P = {};
     int group_bins;
     int64_t chunk_slots, need;
-    // as large as either form of the grid asks for; a folded batch that leaves some unused takes larger chunks
+    // (a folded batch needs no more, and takes fewer chunks where it needs less)
     if (plan_chunks(*desc, false, n_slots, max_bytes, P, group_bins, chunk_slots, need) == 0) return 0;
     return need;
 }

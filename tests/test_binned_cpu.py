@@ -1,0 +1,55 @@
+"""The binned scatter's workspace plan (host arithmetic, no kernel runs): a size that nect_grid_binned_workspace returns is
+one that it, and the launches of both forms of the grid, accept."""
+import ctypes
+import random
+
+import pytest
+import torch
+
+from nect_amd import _lib
+from nect_amd.grid import GridDesc
+
+
+def cases():
+    rng = random.Random(5)
+    yield GridDesc(3, 19, 4, 21, 8, 1.26), 304352, 16 << 20
+    yield GridDesc(4, 16, 2, 15, 5, 1.5), 1 << 15, 1 << 30
+    for _ in range(400):
+        D, F, L, base = rng.choice([3, 4]), rng.choice([2, 4]), rng.randint(1, 32), rng.randint(2, 32)
+        finest = 2 ** (5 + 13 * rng.random())
+        grid = GridDesc(D, L, F, rng.randint(8, 22), base, max(1.0, (finest / base) ** (1 / max(1, L - 1))))
+        yield grid, int(2 ** (5 + 16 * rng.random())), int(2 ** (18 + 16 * rng.random()))
+
+
+def test_a_returned_size_is_accepted():
+    lib = _lib.lib()
+    some = 0
+    for grid, slots, limit in cases():
+        need = lib.nect_grid_binned_workspace(grid.struct_ref(), slots, limit)
+        assert 0 <= need <= limit
+        if need:
+            some += 1
+            again = lib.nect_grid_binned_workspace(grid.struct_ref(), slots, need)
+            assert again == need, (grid.n_dims, grid.n_levels, slots, limit, need, again)
+    assert some > 200
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="hands the entry points host addresses: only where nothing can run")
+def test_launches_accept_a_returned_size():
+    """Without a device a launch fails; it has to get that far (the plan is checked before)."""
+    lib = _lib.lib()
+    at = ctypes.c_void_p(1 << 20)
+    for grid, slots, limit in cases():
+        slots = (slots + 31) // 32 * 32
+        need = lib.nect_grid_binned_workspace(grid.struct_ref(), slots, limit)
+        if not need:
+            continue
+        D, LF = grid.n_dims, grid.n_output_dims
+        told = []
+        for cols in ([0, 1, 2, 3][:D], [0, 1, 3] if D == 3 else [3, 0, 1, 2]):
+            told.append(lib.nect_grid_backward_binned_rays(
+                grid.struct_ref(), (ctypes.c_int32 * D)(*cols), at, at, at, at, slots // 32, 0.5, _lib.F32, at, LF, None, at,
+                at, need, None))
+            assert told[-1] != 0 and b"workspace" not in lib.nect_last_error(), (D, slots, limit, lib.nect_last_error())
+        assert lib.nect_grid_backward_binned(grid.struct_ref(), at, slots, D, _lib.F32, at, LF, None, at, at, need, None) != 0
+        assert b"workspace" not in lib.nect_last_error(), (D, slots, limit, lib.nect_last_error())
