@@ -129,7 +129,7 @@ class BinnedScatter:
         self._sizes: dict = {}
 
     def _need(self, grids, slots: int) -> int:
-        key = (slots, *[(g.n_dims, g.n_levels, g.n_features, g.n_params, g.struct.base_resolution) for g in grids])
+        key = (slots, *[bytes(g.struct) for g in grids])
         need = self._sizes.get(key)
         if need is None:
             each = [int(_lib.lib().nect_grid_binned_workspace(g.struct_ref(), slots, self.max_bytes)) for g in grids]

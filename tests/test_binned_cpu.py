@@ -53,3 +53,18 @@ def test_launches_accept_a_returned_size():
             assert told[-1] != 0 and b"workspace" not in lib.nect_last_error(), (D, slots, limit, lib.nect_last_error())
         assert lib.nect_grid_backward_binned(grid.struct_ref(), at, slots, D, _lib.F32, at, LF, None, at, at, need, None) != 0
         assert b"workspace" not in lib.nect_last_error(), (D, slots, limit, lib.nect_last_error())
+
+
+def test_sizes_are_kept_per_level_table():
+    """Two grids of the same dimensions, parameter count and base resolution, one with a hashed level where the other's is
+    dense (lists of another capacity): each gets its own size."""
+    from nect_amd.fused import BinnedScatter
+
+    dense, hashed = GridDesc(3, 2, 4, 12, 16, 1.0), GridDesc(3, 2, 4, 12, 16, 2.0)
+    assert dense.n_params == hashed.n_params
+    slots = 1 << 22
+    own = [BinnedScatter("cpu", 12 << 30)._need([g], slots) for g in (dense, hashed)]
+    assert own[0] > own[1] > 0
+    for order in ((dense, hashed), (hashed, dense)):
+        kept = BinnedScatter("cpu", 12 << 30)
+        assert {g: kept._need([g], slots) for g in order} == dict(zip((dense, hashed), own))
