@@ -121,6 +121,11 @@ class BinnedScatter:
     # 16 x 2 3-D, 2^19 entries 61 / 59, 118 / 77, 232 / 89 us; 19 x 4, 2^21 entries 100 / 128, 188 / 147, 376 / 223;
     # 16 x 2 4-D, 2^21 entries 117 / 110, 229 / 165, 453 / 231.
     MIN_SLOTS = 1 << 14
+    # Chunks of a workspace of at least this many bytes are large enough; in a smaller one (under a memory budget, or
+    # where the device has little left) a chunk has to hold 2 MIN_SLOTS and 1/2048 of the parameters, too.  Steps of
+    # 2^24 samples, direct / binned: 16 x 2 3-D, 2^19 entries, chunks of 28 k samples 37 / 41 ms, of 112 k 33 / 19;
+    # 4-D, 2^21 entries, of 56 k 68 / 54.
+    AMPLE_BYTES = 2 << 30
 
     def __init__(self, device, max_bytes: int):
         self.device = device
@@ -129,30 +134,47 @@ class BinnedScatter:
         self._sizes: dict = {}
 
     def _need(self, grids, slots: int) -> int:
-        key = (slots, *[bytes(g.struct) for g in grids])
+        """Bytes for a batch of ``slots`` samples within max_bytes; 0 where the grids do not suit, or where the
+        batch would be cut into chunks of too few samples."""
+        key = (slots, self.max_bytes, *[bytes(g.struct) for g in grids])
         need = self._sizes.get(key)
         if need is None:
-            each = [int(_lib.lib().nect_grid_binned_workspace(g.struct_ref(), slots, self.max_bytes)) for g in grids]
-            need = max(each) if each and min(each) > 0 else 0
+            size = _lib.lib().nect_grid_binned_workspace
+            need = 0
+            for g in grids:
+                n = int(size(g.struct_ref(), slots, self.max_bytes))
+                if n > 0 and self.max_bytes < self.AMPLE_BYTES:
+                    chunks = -(-int(size(g.struct_ref(), slots, 1 << 62)) // n)
+                    if chunks > 1 and slots < chunks * max(2 * self.MIN_SLOTS, g.n_params >> 11):
+                        n = 0
+                if n <= 0:
+                    need = 0
+                    break
+                need = max(need, n)
             if len(self._sizes) > 64:
                 self._sizes.clear()
             self._sizes[key] = need
         return need
 
     def suits(self, grids, slots: int) -> bool:
-        """Whether batches of ``slots`` samples take the binned schedule (every grid, one after another)."""
-        return (slots >= self.MIN_SLOTS and all(slots >= g.n_params >> 11 for g in grids)
-                and self._need(grids, slots) > 0)
-
-    def reserve(self, grids, slots: int):
-        need = self._need(grids, slots)
-        if self._buffer is None or self._buffer.numel() < need:
+        """Whether batches of ``slots`` samples take the binned schedule (every grid, one after another); their
+        workspace is then held.  Where the device has not that much left, less is asked for from then on, down to
+        none: the direct schedules need no workspace."""
+        if not grids or slots < max(self.MIN_SLOTS, *[g.n_params >> 11 for g in grids]):
+            return False
+        while (need := self._need(grids, slots)) > 0:
+            if self._buffer is not None and self._buffer.numel() >= need:
+                return True
             self._buffer = None   # the old one is returned before the new one is taken
-            self._buffer = torch.empty(need, dtype=torch.uint8, device=self.device)
+            try:
+                self._buffer = torch.empty(need, dtype=torch.uint8, device=self.device)
+                return True
+            except torch.cuda.OutOfMemoryError:
+                self.max_bytes = need // 2
+        return False
 
-    def workspace(self, grids, slots: int) -> tuple[int, int]:
-        """(pointer, bytes) for a batch of ``slots`` samples."""
-        self.reserve(grids, slots)
+    def workspace(self) -> tuple[int, int]:
+        """(pointer, bytes) for the batch that ``suits`` was last asked about."""
         return self._buffer.data_ptr(), self._buffer.numel()
 
 
@@ -284,8 +306,7 @@ class FusedTrainStep:
         self.loss_value = torch.empty(1, dtype=torch.float32, device=dev)
         ws = int(_lib.lib().nect_mlp_backward_workspace(self.mlp.struct_ref(), _lib.dtype_code(self.dtype), slots))
         self.workspace = torch.empty(max(ws, 16), dtype=torch.uint8, device=dev)
-        if self._use_bins(slots):
-            self._bins.reserve([self.grid], slots)
+        self._use_bins(slots)   # holds the workspace
 
     @property
     def mlp_weights(self) -> torch.Tensor:
@@ -480,7 +501,7 @@ class FusedTrainStep:
         rays = self.rays[:num_rays]
         grad = self.grad[self.n_mlp:].data_ptr()
         if self._use_bins(max_tiles * 32):
-            ws, ws_bytes = self._bins.workspace([self.grid], max_tiles * 32)
+            ws, ws_bytes = self._bins.workspace()
             self._call("grid_backward", "nect_grid_backward_binned_rays", self.grid.struct_ref(), None, _lib.ptr(rays),
                        _lib.ptr(self.tile_offsets), _lib.ptr(self.tile_ray), _lib.ptr(self.n_tiles), int(max_tiles),
                        float(t), _lib.F32, _lib.ptr(self.dfeat), F, None, grad, ws, ws_bytes, st)

@@ -221,7 +221,7 @@ class ModuleTrainStep:
         esz = dfeat.element_size()
         max_tiles = cs.tiles_needed(num_rays, points_per_ray)
         if self._use_bins(max_tiles * 32):
-            ws, ws_bytes = self._bins.workspace(self._grids(), max_tiles * 32)
+            ws, ws_bytes = self._bins.workspace()
             for part, src in zip(self.model.net.grid_parts(), self.model.grid_sources):
                 cols = (ctypes.c_int32 * len(src))(*src)
                 _lib.call("nect_grid_backward_binned_rays", part.desc.struct_ref(), cols, _lib.ptr(rays),

@@ -188,8 +188,8 @@ def _encode_backward(parts: list[_Part], x: torch.Tensor, dfeat: torch.Tensor, g
     if x.shape[0] >= BinnedScatter.MIN_SLOTS:
         grids = [p for p in parts if p.kind == "grid"]
         bins = BinnedScatter(x.device, POINTS_SCATTER_BYTES)
-        if grids and bins.suits([p.desc for p in grids], x.shape[0]):
-            ws, ws_bytes = bins.workspace([p.desc for p in grids], x.shape[0])
+        if bins.suits([p.desc for p in grids], x.shape[0]):
+            ws, ws_bytes = bins.workspace()
             for p in grids:
                 _lib.call("nect_grid_backward_binned", p.desc.struct_ref(), _lib.ptr(x) + 4 * p.col0, x.shape[0],
                           x.shape[1], _lib.F32, dfeat.data_ptr() + 4 * p.out0, dfeat.stride(0), None,
