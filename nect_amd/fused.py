@@ -131,7 +131,14 @@ class BinnedScatter:
         self.device = device
         self.max_bytes = int(max_bytes)
         self._buffer: torch.Tensor | None = None
+        self._lent: torch.Tensor | None = None
         self._sizes: dict = {}
+
+    def lend(self, buffer: torch.Tensor):
+        """Records go into ``buffer`` (which holds nothing between the owner's forward passes), and no memory of
+        their own is taken."""
+        self._lent, self._buffer = buffer, None
+        self.max_bytes = buffer.numel() * buffer.element_size()
 
     def _need(self, grids, slots: int) -> int:
         """Bytes for a batch of ``slots`` samples within max_bytes; 0 where the grids do not suit, or where the
@@ -163,7 +170,7 @@ class BinnedScatter:
         if not grids or slots < max(self.MIN_SLOTS, *[g.n_params >> 11 for g in grids]):
             return False
         while (need := self._need(grids, slots)) > 0:
-            if self._buffer is not None and self._buffer.numel() >= need:
+            if self._lent is not None or (self._buffer is not None and self._buffer.numel() >= need):
                 return True
             self._buffer = None   # the old one is returned before the new one is taken
             try:
@@ -175,7 +182,8 @@ class BinnedScatter:
 
     def workspace(self) -> tuple[int, int]:
         """(pointer, bytes) for the batch that ``suits`` was last asked about."""
-        return self._buffer.data_ptr(), self._buffer.numel()
+        held = self._lent if self._lent is not None else self._buffer
+        return held.data_ptr(), held.numel() * held.element_size()
 
 
 class FusedTrainStep:
@@ -186,8 +194,8 @@ class FusedTrainStep:
                  weight_decay: float = 0.0, memory_budget: int | None = None):
         """``memory_budget`` (bytes) bounds the per-sample buffers (features, their gradients, mu, dmu): a batch
         whose samples exceed it is processed in chunks of rays that fit, each chunk's gradient weighted by its
-        share of the batch, and one optimiser step at the end.  It also bounds the table gradient's record
-        workspace, which is a buffer of its own."""
+        share of the batch, and one optimiser step at the end.  The table gradient's record workspace lies within
+        the budget: in what these buffers leave of it or, where that is less, in the features' memory."""
         if mlp.n_input != grid.n_output_dims:
             raise ValueError("MLP input width must equal the grid's L*F")
         if params.dtype != torch.float32 or not params.is_cuda:
@@ -238,8 +246,7 @@ class FusedTrainStep:
         self.scatter_split = False
         self._order_ws = torch.empty(0, dtype=torch.uint8, device=self.device)
         self._order_need: dict = {}
-        self._bins = BinnedScatter(self.device, BinnedScatter.MAX_BYTES if memory_budget is None
-                                   else min(BinnedScatter.MAX_BYTES, memory_budget))
+        self._bins = BinnedScatter(self.device, BinnedScatter.MAX_BYTES)
         self._plan_cache: dict = {}
         self._chunk_counts: list = []
         self._alloc(max_rays, max_points_per_ray)
@@ -306,6 +313,13 @@ class FusedTrainStep:
         self.loss_value = torch.empty(1, dtype=torch.float32, device=dev)
         ws = int(_lib.lib().nect_mlp_backward_workspace(self.mlp.struct_ref(), _lib.dtype_code(self.dtype), slots))
         self.workspace = torch.empty(max(ws, 16), dtype=torch.uint8, device=dev)
+        if self.memory_budget is not None:
+            # within the budget: what the per-sample buffers leave of it, or the features' memory, which holds nothing
+            # from the network's backward to the next encoding, whichever is more
+            spare = self.memory_budget - chunk * per_ray
+            self._bins = BinnedScatter(dev, min(BinnedScatter.MAX_BYTES, max(spare, 0)))
+            if spare < self.features.numel() * self.features.element_size():
+                self._bins.lend(self.features)
         self._use_bins(slots)   # holds the workspace
 
     @property

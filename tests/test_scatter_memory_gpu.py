@@ -1,5 +1,5 @@
 """The memory of the table gradient's records: where the device has not enough left for them, every training path works
-with less or none, as it does with plenty.
+with less or none, as it does with plenty; a fused step's memory budget holds for them, too.
 
 The gradients are the same sums in another order: 1e-4 of the largest (as for batches in chunks)."""
 import contextlib
@@ -85,6 +85,30 @@ def test_fused_step_with_little_memory(device, left):
         assert torch.equal(fs.y_pred, y)
         same(fs.grad, ref)
         assert fs._bins._buffer is None or fs._bins._buffer.numel() < left * MIB
+
+
+def test_fused_step_memory_budget(device):
+    """A batch that the budget cuts in two, one that it leaves no room beside and one that it leaves some: the records lie
+    within it, and the gradient is that without a budget."""
+    B, S = 16384, 128
+    b = batch(device, B)
+    fs = fused(device, B, S, b)
+    ref, per_ray = fs.grad.clone(), fs.slot_bytes() * S
+    del fs
+    fixed = None
+    for rays, spare, own in [(B // 2, 0, False), (B, 0, False), (B, 1 << 30, True)]:
+        budget = per_ray * rays + spare
+        print(f"[memory] budget {budget / MIB:.0f} MiB", flush=True)
+        fs, used = peak(device, lambda: fused(device, B, S, b, memory_budget=budget))
+        assert fs.chunk_rays == rays
+        same(fs.grad, ref)
+        assert fs._use_bins(rays * S)
+        assert (fs._bins._buffer is not None) == own
+        # beside the budget: parameters, rays and the like, the same for all
+        fixed = used - budget if fixed is None else fixed
+        assert used <= budget + fixed + 64 * MIB, (used, budget, fixed)
+        assert fixed < 400 * MIB
+        del fs
 
 
 def test_module_step_with_little_memory(device):
