@@ -42,7 +42,9 @@ class ModuleTrainStep:
 
     def __init__(self, model: torch.nn.Module, dtype: torch.dtype, max_rays: int, max_points_per_ray: int,
                  loss: str = "L2", betas=(0.9, 0.999), eps: float = 1e-8, weight_decay: float = 0.0,
-                 dynamic: bool = False):
+                 dynamic: bool = False, scatter_bytes: int = BinnedScatter.MAX_BYTES):
+        """``scatter_bytes``: most memory the step holds for the table gradient's records (0: none, the gradient
+        is scattered straight to the table)."""
         self.model = model
         self.params = model.net.params
         if self.params.dtype != torch.float32 or not self.params.is_cuda:
@@ -67,7 +69,7 @@ class ModuleTrainStep:
         # table-gradient schedule when the model names its grids' coordinates: "bins" (records sorted by table part)
         # or "groups" (ray groups); "module" leaves it to the module's own backward
         self.scatter = "bins" if getattr(model, "grid_sources", None) is not None else "module"
-        self._bins = BinnedScatter(self.device, BinnedScatter.MAX_BYTES)
+        self._bins = BinnedScatter(self.device, scatter_bytes)
         self.presort = True
         self.agg_rounds: list | None = None      # per grid, per level; None: aggregation_plan()
         # the scatter's launches (nect_grid_backward_ray_groups' split): 0 one launch per grid, 1 the aggregated

@@ -1,5 +1,5 @@
 """The memory of the table gradient's records: where the device has not enough left for them, every training path works
-with less or none, as it does with plenty; a fused step's memory budget holds for them, too.
+with less or none, as it does with plenty; a fused step's memory budget holds for them, too; a module step's can be set.
 
 The gradients are the same sums in another order: 1e-4 of the largest (as for batches in chunks)."""
 import contextlib
@@ -124,17 +124,17 @@ def test_module_step_with_little_memory(device):
            "n_hidden_layers": 2}
     m = QuadCubes(enc, net, include_identity=True, dtype=torch.float16, seed=4).to(device)
 
-    def run(scatter="bins"):
-        st = ModuleTrainStep(m, torch.float16, B, S, loss="L2", dynamic=True)
+    def run(**kw):
+        st = ModuleTrainStep(m, torch.float16, B, S, loss="L2", dynamic=True, **kw)
         st.GROUPS_MIN_WORKGROUPS = 0
-        st.scatter = scatter
         st.step(geo, 0.8, idx, 0, B, S, l_max / S, True, jit, off, tgt, l_max, lr=0.0, t=0.6, optimizer_step=False)
         return st
 
     st = run()
     ref, want = st.grad.clone(), st._bins._buffer.numel()
     del st
-    st, used = peak(device, lambda: run("groups"))
+    st, used = peak(device, lambda: run(scatter_bytes=0))
+    assert not st._use_bins(B * S) and st._bins._buffer is None
     same(st.grad, ref)
     del st
     assert want > 256 * MIB
