@@ -441,6 +441,35 @@ def test_benchmarked_step_matches_oracle_at_its_shape(device, name):
         assert e < gtol, (part, e)
 
 
+@pytest.fixture
+def ray_groups(monkeypatch):
+    """The large-batch schedule in patch order through the ray-group scatter, which batches take that binned records do
+    not suit."""
+    from nect_amd.fused import BinnedScatter, FusedTrainStep
+
+    took = []
+    order = FusedTrainStep._ray_order
+
+    def ray_order(self, geometry, ray_index, start, num_rays, points_per_ray):
+        took.append(self._use_groups(num_rays, points_per_ray))
+        return order(self, geometry, ray_index, start, num_rays, points_per_ray)
+
+    monkeypatch.setattr(BinnedScatter, "suits", lambda self, grids, slots: False)
+    monkeypatch.setattr(FusedTrainStep, "_ray_order", ray_order)
+    yield
+    assert took and all(took)
+
+
+@pytest.mark.parametrize("name", list(BENCH_STEPS))
+def test_benchmarked_step_through_ray_groups(device, name, ray_groups):
+    test_benchmarked_step_matches_oracle_at_its_shape(device, name)
+
+
+def test_accumulated_and_chunked_steps_through_ray_groups(device, ray_groups):
+    test_continuous_scanning_step_matches_oracle(device, torch.float32, "L2", True)
+    test_memory_budget_chunks_match_one_pass(device, torch.float16, True)
+
+
 def test_fp16_step_skips_non_finite_gradient_and_backs_off(device):
     """precision="16-mixed" semantics on the device: a batch whose gradient is not finite (an Inf target) leaves
     params, m, v and the fp16 copy bit-unchanged, zeroes the gradient, halves the loss scale and does not count
