@@ -38,6 +38,7 @@
 // the same sum over the samples: the records are formed over the other
 // dimensions only (half as many), summed, and each sum is added to both entries.
 #include <algorithm>
+#include <type_traits>
 
 #include "sources.hpp"
 
@@ -678,9 +679,15 @@ static bool level_is_hashed(const NectGridDesc &g, int l) {
     return stride > g.level_size[l];
 }
 
+// Runs of 2^granule table entries along the first coordinate that a slice of a level, its last coordinate held, touches.
+static int64_t runs_per_slice(uint32_t res, int granule) {
+    return (int64_t)res * std::max<int64_t>(1, ((int64_t)res >> granule));
+}
+
 // Fills P for batches of at most `slots` samples per chunk; returns the record
 // buffer's records, or -1 when a level needs more bins than the kernels take.
-static int64_t plan_bins(const NectGridDesc &g, bool fold, int64_t slots, BinPlan &P, int &group_bins) {
+// `points`: a caller's (their number and sizes do not depend on it).
+static int64_t plan_bins(const NectGridDesc &g, bool fold, bool points, int64_t slots, BinPlan &P, int &group_bins) {
     const int dims = g.n_dims - (fold ? 1 : 0);
     const int64_t pairs = slots << (dims - 1);
     // small batches (a few rays, a region) crowd into few bins more often, and lists that hold the whole batch cost
@@ -730,7 +737,16 @@ static int64_t plan_bins(const NectGridDesc &g, bool fold, int64_t slots, BinPla
         group_bins = std::max(group_bins, in_group);
         // (two dimensions: a hashed index holds few values of its second term, which alone would choose the bin)
         const bool spread = hashed && dims > 2 && (size & (size - 1)) == 0;
-        const int gr = lb == 0 || spread ? log2_entries : 6;
+        int gr = lb == 0 || spread ? log2_entries : 6;
+        // A caller's points may all have one last coordinate (a model over (z, y, t) at one time): the second term alone
+        // then chooses the bin here, too, and where it has few values for the bins (four features: twice as many bins,
+        // and a record past its list costs twice the atomics) lists overflow.  Such levels' bins interleave in runs short
+        // enough for four runs of a slice per bin, and no shorter than 64 entries: a pair across two runs adds its second
+        // entry by itself.  A million random points, 16 x 4, T = 2^19: last coordinate held 4.86 -> 1.97 ms (atomics
+        // without records: 5.14), all varying 1.31 -> 1.40; 23 levels of growth 1.17, T = 2^21: 7.91 -> 3.67 (6.67)
+        // and 2.47 -> 2.54.
+        if (points && dims == 3 && g.n_features == 4 && spread && nb >= 256)
+            while (gr > 6 && runs_per_slice(g.resolution[l], gr) < 4 * (int64_t)nb) --gr;
         P.log2_bins[l] = (uint8_t)lb;
         P.granule[l] = (uint8_t)gr;
         const int64_t rows = ((int64_t)size + ((int64_t)1 << (gr + lb)) - 1) >> (gr + lb);
@@ -763,13 +779,13 @@ static int64_t plan_bins(const NectGridDesc &g, bool fold, int64_t slots, BinPla
 
 // Chunks so that counters and records fit in `bytes`; 0 when they cannot.  The counts tried do not depend on `bytes`, so
 // that the size found for one limit is enough for the launch, whose limit it is.
-static int plan_chunks(const NectGridDesc &g, bool fold, int64_t slots, int64_t bytes, BinPlan &P, int &group_bins,
-                       int64_t &chunk_slots, int64_t &need) {
+static int plan_chunks(const NectGridDesc &g, bool fold, bool points, int64_t slots, int64_t bytes, BinPlan &P,
+                       int &group_bins, int64_t &chunk_slots, int64_t &need) {
     const int64_t rec_bytes = 8 + 4 * g.n_features;
     const int64_t tiles = (slots + kTile - 1) / kTile;
     for (int64_t k = 1; k <= tiles && k <= 4096; k += std::max<int64_t>(1, k / 16)) {
         chunk_slots = ((tiles + k - 1) / k) * kTile;
-        const int64_t rec = plan_bins(g, fold, chunk_slots, P, group_bins);
+        const int64_t rec = plan_bins(g, fold, points, chunk_slots, P, group_bins);
         if (rec < 0) return 0;
         need = rec * rec_bytes + k * (int64_t)P.n_counters * P.n_lists * 4;
         if (need <= bytes) {
@@ -787,7 +803,8 @@ static int32_t launch_binned(const NectGridDesc &g, const Src &src, float t, int
     P.t = t;
     int group_bins;
     int64_t chunk_slots, need;
-    const int chunks = plan_chunks(g, FOLD, slots, ws_bytes, P, group_bins, chunk_slots, need);
+    constexpr bool kPoints = std::is_same<Src, PointRowsSource<D>>::value;
+    const int chunks = plan_chunks(g, FOLD, kPoints, slots, ws_bytes, P, group_bins, chunk_slots, need);
     NECT_REQUIRE(chunks > 0, "workspace too small for this grid and batch");
     uint32_t *counts = static_cast<uint32_t *>(ws);
     const int n_counts = chunks * P.n_lists * P.n_counters;
@@ -856,7 +873,7 @@ extern "C" int64_t nect_grid_binned_workspace(const NectGridDesc *desc, int64_t 
     int group_bins;
     int64_t chunk_slots, need;
     // (a folded batch needs no more, and takes fewer chunks where it needs less)
-    if (plan_chunks(*desc, false, n_slots, max_bytes, P, group_bins, chunk_slots, need) == 0) return 0;
+    if (plan_chunks(*desc, false, false, n_slots, max_bytes, P, group_bins, chunk_slots, need) == 0) return 0;
     return need;
 }
 
