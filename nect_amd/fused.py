@@ -116,14 +116,13 @@ class BinnedScatter:
     # Scatter of the 256^3 step (10.7 M samples) with 1.9 / 3.5 / 7 GiB: 6.4 / 6.1 / 5.9 ms; QuadCubes preset step
     # (2^23-entry tables, whose sums cost most to add) with 6 / 12 / 24 GiB: 37.8 / 33.1 / 33.1 ms.
     MAX_BYTES = 12 << 30
-    # Fewer samples than this, or than 1/2048 of the table's parameters, scatter straight to the table: the bins'
-    # sums are cleared and searched whatever the batch.  Direct / binned at 2^14, 2^15, 2^16 random points:
-    # 16 x 2 3-D, 2^19 entries 61 / 59, 118 / 77, 232 / 89 us; 19 x 4, 2^21 entries 100 / 128, 188 / 147, 376 / 223;
-    # 16 x 2 4-D, 2^21 entries 117 / 110, 229 / 165, 453 / 231.
+    # Fewer samples than this, or than least() of the grid, scatter straight to the table.  Direct / binned at 2^14, 2^15,
+    # 2^16 random points: 16 x 2 3-D, 2^19 entries 61 / 59, 118 / 77, 232 / 89 us; 19 x 4, 2^21 entries 100 / 128,
+    # 188 / 147, 376 / 223; 16 x 2 4-D, 2^21 entries 117 / 110, 229 / 165, 453 / 231.
     MIN_SLOTS = 1 << 14
     # Chunks of a workspace of at least this many bytes are large enough; in a smaller one (under a memory budget, or
-    # where the device has little left) a chunk has to hold 2 MIN_SLOTS and 1/2048 of the parameters, too.  Steps of
-    # 2^24 samples, direct / binned: 16 x 2 3-D, 2^19 entries, chunks of 28 k samples 37 / 41 ms, of 112 k 33 / 19;
+    # where the device has little left) a chunk has to hold 2 MIN_SLOTS and least(), too.  Steps of 2^24 samples,
+    # direct / binned: 16 x 2 3-D, 2^19 entries, chunks of 28 k samples 37 / 41 ms, of 112 k 33 / 19;
     # 4-D, 2^21 entries, of 56 k 68 / 54.
     AMPLE_BYTES = 2 << 30
 
@@ -133,6 +132,19 @@ class BinnedScatter:
         self._buffer: torch.Tensor | None = None
         self._lent: torch.Tensor | None = None
         self._sizes: dict = {}
+
+    @staticmethod
+    def least(grid) -> int:
+        """Fewest samples whose scatter the records shorten: the bins' sums are cleared and searched whatever the
+        batch, so it grows with the table, faster where a level has more than 2048 bins (a workgroup's records then
+        find few others of their bin).  Steps of one batch of rays, straight to the table / binned, us: 3-D, two features,
+        2^19 entries 2^14 samples 112 / 123, 2^15 158 / 144; 2^21 2^15 168 / 184, 2^16 272 / 253; 2^23 2^17 473 / 536,
+        2^18 764 / 731.  Four features, 2^20 2^15 202 / 198; 2^21 2^16 338 / 340, 2^17 516 / 469; 2^22 2^16 348 / 415,
+        2^17 526 / 546, 2^18 808 / 762; 2^23 2^19 1531 / 1609, 2^20 2921 / 2684.  4-D, 2^20 2^14 161 / 166, 2^15
+        241 / 214; 2^22 2^16 470 / 453."""
+        bins = grid.struct.level_size[grid.n_levels - 1] * grid.n_features >> 13
+        eighths = 64 if bins > 2048 else (8 if grid.n_dims == 4 else (16 if grid.n_features == 4 else 22))
+        return max(BinnedScatter.MIN_SLOTS, grid.n_params * eighths >> 14)
 
     def lend(self, buffer: torch.Tensor):
         """Records go into ``buffer`` (which holds nothing between the owner's forward passes), and no memory of
@@ -152,7 +164,7 @@ class BinnedScatter:
                 n = int(size(g.struct_ref(), slots, self.max_bytes))
                 if n > 0 and self.max_bytes < self.AMPLE_BYTES:
                     chunks = -(-int(size(g.struct_ref(), slots, 1 << 62)) // n)
-                    if chunks > 1 and slots < chunks * max(2 * self.MIN_SLOTS, g.n_params >> 11):
+                    if chunks > 1 and slots < chunks * max(2 * self.MIN_SLOTS, self.least(g)):
                         n = 0
                 if n <= 0:
                     need = 0
@@ -167,7 +179,7 @@ class BinnedScatter:
         """Whether batches of ``slots`` samples take the binned schedule (every grid, one after another); their
         workspace is then held.  Where the device has not that much left, less is asked for from then on, down to
         none: the direct schedules need no workspace."""
-        if not grids or slots < max(self.MIN_SLOTS, *[g.n_params >> 11 for g in grids]):
+        if not grids or any(slots < self.least(g) for g in grids):
             return False
         while (need := self._need(grids, slots)) > 0:
             if self._lent is not None or (self._buffer is not None and self._buffer.numel() >= need):

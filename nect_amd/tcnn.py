@@ -36,6 +36,10 @@ from .fused import BinnedScatter, xavier_init
 MAX_GRID_PARTS = 5   # NECT_MAX_GRID_PARTS
 # most bytes of records the table gradient of a caller's points takes from torch's allocator for a backward
 POINTS_SCATTER_BYTES = 2 << 30
+# and the most floats of a level's table whose gradient is taken so (2048 bins): with more, samples along rays, which the
+# atomics' schedule sums as they come, are slower (1.25 M samples of a training batch, 23 x 4 grids, 2^23 entries: 3.1 ms
+# straight to the table, 3.8 binned, with one coordinate held 1.8 and 3.9; 2^22 entries 3.0 and 2.6, 1.8 and 2.2)
+POINTS_SCATTER_FLOATS = 1 << 24
 
 
 def torch_activation(name: str | None, z: torch.Tensor) -> torch.Tensor:
@@ -185,8 +189,9 @@ def _encode_backward(parts: list[_Part], x: torch.Tensor, dfeat: torch.Tensor, g
         return
     if dfeat.stride(1) != 1:
         dfeat = dfeat.contiguous()
-    if x.shape[0] >= BinnedScatter.MIN_SLOTS:
-        grids = [p for p in parts if p.kind == "grid"]
+    grids = [p for p in parts if p.kind == "grid"]
+    if x.shape[0] >= BinnedScatter.MIN_SLOTS and all(p.desc.struct.level_size[p.desc.n_levels - 1] * p.desc.n_features
+                                                     <= POINTS_SCATTER_FLOATS for p in grids):
         bins = BinnedScatter(x.device, POINTS_SCATTER_BYTES)
         if bins.suits([p.desc for p in grids], x.shape[0]):
             ws, ws_bytes = bins.workspace()

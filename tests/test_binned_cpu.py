@@ -68,3 +68,18 @@ def test_sizes_are_kept_per_level_table():
     for order in ((dense, hashed), (hashed, dense)):
         kept = BinnedScatter("cpu", 12 << 30)
         assert {g: kept._need([g], slots) for g in order} == dict(zip((dense, hashed), own))
+
+
+# (grid, samples, whether the records' schedule was the faster one by more than 5 % either way: the measured steps that
+# BinnedScatter.least lists, and a dynamic preset's training batches)
+@pytest.mark.parametrize("args,slots,binned", [
+    ((3, 16, 2, 19, 16, 1.5), 1 << 14, False), ((3, 16, 2, 19, 16, 1.5), 1 << 15, True),
+    ((3, 16, 2, 21, 16, 1.5), 1 << 15, False), ((3, 16, 2, 21, 16, 1.5), 1 << 16, True),
+    ((3, 16, 2, 23, 16, 1.5), 1 << 17, False), ((3, 19, 4, 21, 8, 1.26), 1 << 17, True),
+    ((3, 19, 4, 22, 8, 1.26), 1 << 16, False), ((3, 19, 4, 23, 8, 1.26), 1 << 19, False),
+    ((3, 19, 4, 23, 8, 1.26), 1 << 20, True), ((4, 16, 2, 20, 16, 1.5), 1 << 15, True),
+    ((3, 23, 4, 23, 16, 1.17), 1_000_000, False), ((3, 23, 4, 23, 16, 1.17), 2_499_840, True)])
+def test_batches_take_the_faster_schedule(args, slots, binned):
+    from nect_amd.fused import BinnedScatter
+
+    assert (slots >= BinnedScatter.least(GridDesc(*args))) == binned
