@@ -33,11 +33,19 @@ __device__ __forceinline__ float rescale_value(const NectQueryJob &J, float mu) 
     return (float)h;
 }
 
+// Whether z-neighbours are close enough for the stacked order: up to eight times the others' spacing (the server's rule).
+__device__ __forceinline__ bool fine_along_z(const NectQueryJob &J) {
+    float step[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) step[k] = fabsf(J.b[k] - J.a[k]) / (float)max(J.n[k] - 1, 1);
+    return step[0] <= 8.0f * fmaxf(step[1], step[2]);
+}
+
 // Voxel (iz, iy, ix) at traversal position v of a job's grid; false for positions
 // in the padding or past the grid.  Row order, or (J.brick) the grid padded to
 // whole bricks of 2^lz x 2^ly x 2^lx voxels: in row order, their voxels in row
-// order, or (NECT_BRICK_STACKED, and a job that takes the whole traversal, where
-// the order is nobody's business) in layers of bricks stacked up to 32 voxels
+// order, or (NECT_BRICK_STACKED, and a finely spaced job that takes the whole
+// traversal, where the order is nobody's business) in layers of bricks stacked up to 32 voxels
 // along z; a layer column by column, a column (one stack of bricks) with z
 // fastest, then x, then y.
 // z is the grid's first coordinate, whose neighbouring cells are neighbouring
@@ -66,7 +74,8 @@ __device__ __forceinline__ bool query_voxel(const NectQueryJob &J, int64_t v, in
     const uint32_t nby = ((uint32_t)J.n[1] + (1u << ly) - 1u) >> ly;
     const uint32_t nbz = ((uint32_t)J.n[0] + (1u << lz) - 1u) >> lz;
     const uint32_t plane = nby * nbx;
-    if (!(J.brick & NECT_BRICK_STACKED) && (J.v0 != 0 || J.count < ((int64_t)(nbz * plane) << ib))) {
+    if (!(J.brick & NECT_BRICK_STACKED) &&
+        (J.v0 != 0 || J.count < ((int64_t)(nbz * plane) << ib) || !fine_along_z(J))) {
         const uint32_t bz = b / plane;
         const uint32_t r = b - bz * plane;
         const uint32_t by = r / nbx;

@@ -80,6 +80,14 @@ class QueryRequest:
     def voxels(self) -> int:
         return int(self.n[0]) * int(self.n[1]) * int(self.n[2])
 
+    def fine_along_z(self) -> bool:
+        """Whether voxels that follow one another along z are close enough to share cache lines of the table.  A layer of
+        512^2 voxels, 32 of them, 4-D BF16 model with 2^21 entries, by z spacing over x spacing (1/1023, 1/511): bricks in
+        row order / stacked along z at 1 3.0 / 1.6, 4.4 / 1.8 ms; at 4 4.0 / 2.6, 6.0 / 4.4; at 8 4.9 / 4.2, 6.7 / 6.1; at
+        16 5.5 / 5.9; at 32 5.9 / 7.2."""
+        step = [abs(b - a) / max(k - 1, 1) for k, a, b in zip(self.n, self.a, self.b)]
+        return step[0] <= 8 * max(step[1], step[2])
+
     @property
     def latency(self) -> float | None:
         return None if self.done is None else self.done - self.arrival
@@ -214,7 +222,7 @@ class QueryServer:
             jobs[k]["lo"] = r.lo
             jobs[k]["mu_dtype"] = _lib.F16 if r.mu_half else _lib.F32
             jobs[k]["rescale"] = r.rescale
-            jobs[k]["brick"] = r.brick | BRICK_STACKED if r.brick else 0
+            jobs[k]["brick"] = r.brick | BRICK_STACKED if r.brick and r.fine_along_z() else r.brick
             if r.axes is not None:
                 for d in range(3):
                     ax = r.axes[d]
