@@ -198,7 +198,9 @@ static unsigned query_blocks(const void *kernel, int threads, size_t lds_bytes, 
         per_cu <= 0)
         per_cu = 2;
     const int64_t resident = (int64_t)query_cus() * per_cu;
-    int64_t b = std::min<int64_t>(needed, resident);
+    // (as many as share the tiles out evenly over the rounds)
+    const int64_t rounds = (needed + resident - 1) / resident;
+    int64_t b = (needed + rounds - 1) / rounds;
     b = (b + kXcds - 1) / kXcds * kXcds;
     return (unsigned)std::max<int64_t>(b, kXcds);
 }
