@@ -130,11 +130,11 @@ __global__ __launch_bounds__(64 * kTwinWaves, 1) void k_mlp_backward_shared(MlpA
     };
     chunk x[NT];
     float dy = 0.0f;
-    // rows past the last tile's last one read that one; their dL/dz is zero.  (Not the rows between the count on the
-    // device and a.n: they may never have been written, and zero times what they hold is not zero where that is not finite.)
-    const int64_t last = min(n_tiles * kTile, a.n) - 1;
+    // rows past the end read the last one, a tile past the last one that one; their dL/dz is zero.  (Not the rows between
+    // the count on the device and a.n: they may never have been written, and zero times what they hold is not zero where
+    // that is not finite.)
     const auto fetch = [&](int64_t tile) {
-        const int64_t row = min(tile * kTile + s0, last);
+        const int64_t row = min(min(tile, n_tiles - 1) * kTile + s0, a.n - 1);
         const T *xr = input_row<T>(a, row);
         if (pieces) {
 #pragma unroll
