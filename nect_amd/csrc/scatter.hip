@@ -109,9 +109,10 @@ struct PointRowsSource {
 
 // Per level: 2^bins bins of `entries` table entries each; entry i belongs to bin
 // (i >> granule) mod 2^bins.  A hashed level's bins are contiguous (its entries
-// are spread evenly anyway, and a pair almost never straddles two); a dense
-// level's interleave in runs of 2^granule entries, so that a batch confined to a
-// part of the volume or to one time still uses every bin.
+// are spread evenly anyway, and a pair almost never straddles two; but see
+// plan_bins for a caller's points); a dense level's interleave in runs of
+// 2^granule entries, so that a batch confined to a part of the volume or to one
+// time still uses every bin.
 struct BinPlan {
     int32_t n_chunks;
     uint32_t hashed;                  // bit l: level l is hashed

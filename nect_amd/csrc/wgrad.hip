@@ -6,10 +6,10 @@
 // one 128 x 128 output tile on MFMA and adds its partial tile to dW with float
 // atomics (16 consecutive floats of a row per 64-byte request).
 //
-// Reading both operands once bounds it: 2.5 M samples of 128 x 128, 1.28 GB, in 235 us.  The operands are staged in LDS as
+// Reading both operands once bounds it: 2.5 M samples of 128 x 128, 1.28 GB, in 227 us.  The operands are staged in LDS as
 // they lie in memory, by 16-byte loads, and turned by the LDS reads (ds_read_b64_tr_b16); two workgroups per CU take one
 // chunk each, since every chunk costs a tile of atomics.  Before, 2-byte loads turned the operands on the way into LDS, in
-// 4096 chunks: 419 us; 300000 samples of 128 x 128 98 -> 53 us, of 128 x 384 322 -> 105.
+// 4096 chunks: 390 us; 300000 samples of 128 x 128 94 -> 50 us, of 128 x 384 297 -> 91.
 #include <algorithm>
 
 #include "mlp_bwd.hpp"
